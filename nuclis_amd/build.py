@@ -16,7 +16,8 @@ from pathlib import Path
 PKG = Path(__file__).resolve().parent
 CSRC = PKG / "csrc"
 LIB = PKG / "libnuq.so"
-SOURCES = ["api.hip", "gemv.hip", "gemv_int.hip", "gemm.hip", "sampling.hip", "quantize.cpp", "gguf.cpp"]
+SOURCES = ["api.hip", "gemv.hip", "gemv_int.hip", "gemm.hip", "panel_plan.hip", "sampling.hip", "quantize.cpp", "gguf.cpp"]
+PANEL_ENCODINGS = [23, 13, 14, 12, 8]  # panel.hip is compiled once per encoding
 ARCH = "gfx950"
 
 
@@ -31,12 +32,14 @@ def build(verbose: bool = False) -> Path:
     common = ["-O3", "-std=c++17", "-fPIC", "-Wall", "-Wno-unused-function", "-I", str(PKG.parent / "include")]
     objects = []
     procs = []
-    for src in SOURCES:
-        obj = build_dir / (Path(src).stem + ".o")
+    units = [("panel.hip", f"panel_{e}.o", [f"-DPANEL_ENC={e}"]) for e in PANEL_ENCODINGS]
+    units += [(src, Path(src).stem + ".o", []) for src in SOURCES]
+    for src, name, defines in units:
+        obj = build_dir / name
         if src.endswith(".hip"):
             cmd = [hipcc(), "-x", "hip", f"--offload-arch={ARCH}", *common,
                    "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
-                   "-fno-gpu-flush-denormals-to-zero", "-munsafe-fp-atomics",
+                   "-fno-gpu-flush-denormals-to-zero", "-munsafe-fp-atomics", *defines,
                    "-c", str(CSRC / src), "-o", str(obj)]
         else:
             cmd = [hipcc(), *common, "-pthread", "-c", str(CSRC / src), "-o", str(obj)]

@@ -229,8 +229,8 @@ int run_gemv(nuq_context *ctx, const nuq_matrix *m, uint64_t stride, const float
 int run_rows_mfma(nuq_context *ctx, const nuq_matrix *m, uint64_t stride, const float *x, uint64_t in_stride,
                   float *out, uint64_t out_stride, uint32_t tokens) {
     if (tokens < 2 || tokens > 8 || (m->encoding != NUQ_Q4_K && m->encoding != NUQ_Q5_K)) return -1;
-    (void)ensure_workspace(ctx, nuq::tile_workspace_floats(m->encoding, (uint32_t)m->rows, (uint32_t)m->columns,
-                                                           std::min(tokens, 4u), in_stride, true));
+    (void)ensure_workspace(ctx, nuq::verify_workspace_floats(m->encoding, (uint32_t)m->rows, (uint32_t)m->columns,
+                                                             std::min(tokens, 4u), true));
     for (uint32_t t0 = 0; t0 < tokens;) {
         const uint32_t c = std::min(tokens - t0, 4u);
         bool taken = false;
@@ -313,11 +313,19 @@ int matmul_impl(nuq_context *ctx, uint32_t kernel, const nuq_matrix *m, const vo
                                           (uint32_t)m->rows, (uint32_t)m->columns, x, f16, in_stride, out,
                                           out_stride, tokens),
                          "multi-token gemv launch");
-    (void)ensure_workspace(ctx, nuq::tile_workspace_floats(m->encoding, (uint32_t)m->rows, (uint32_t)m->columns,
-                                                           tokens, in_stride));
+    nuq::TilePlan plan;
+    const auto plan_with = [&](uint64_t floats) {
+        nuq::plan_tile(m->encoding, (uint32_t)m->rows, (uint32_t)m->columns, tokens, f16, stride, in_stride, floats,
+                       &plan);
+    };
+    plan_with(UINT64_MAX);
+    // without the workspace it wants (a capture, no memory), what the present
+    // one serves
+    if (!ensure_workspace(ctx, plan.floats)) plan_with((uint64_t)ctx->split.tiles * 256 * 256);
     return hip_check(ctx,
                      nuq::launch_tile(ctx->stream, m->encoding, (const uint8_t *)m->bytes, stride, (uint32_t)m->rows,
-                                      (uint32_t)m->columns, x, f16, in_stride, out, out_stride, tokens, ctx->split),
+                                      (uint32_t)m->columns, x, f16, in_stride, out, out_stride, tokens, plan,
+                                      ctx->split),
                      "tile launch");
 }
 

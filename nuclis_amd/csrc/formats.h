@@ -172,10 +172,11 @@ __device__ __forceinline__ float decode_value(uint32_t encoding, const uint8_t *
 // v_perm_b32 pick from table entries 0-7 and 8-15 (selectors 0-7 address the
 // eight bytes of a dword pair, low dword first); a third picks byte e of
 // the second when bit 3 of code e is set (selector e + 4), else of the first
-// (selector e).
+// (selector e). X is folded into the table (result ^ X).
+template <uint32_t X = 0>
 __device__ __forceinline__ uint32_t iq4_lookup(uint32_t codes) {
     // entries 0-3, 4-7, 8-11, 12-15 of kIq4Values as little-endian bytes
-    constexpr uint32_t T0 = 0xbfad9881u, T1 = 0xf6eaddcfu, T2 = 0x26190d01u, T3 = 0x71594535u;
+    constexpr uint32_t T0 = 0xbfad9881u ^ X, T1 = 0xf6eaddcfu ^ X, T2 = 0x26190d01u ^ X, T3 = 0x71594535u ^ X;
     const uint32_t sel = codes & 0x07070707u;
     const uint32_t lo = __builtin_amdgcn_perm(T1, T0, sel), hi = __builtin_amdgcn_perm(T3, T2, sel);
     const uint32_t pick = ((codes >> 1) & 0x04040404u) | 0x03020100u;

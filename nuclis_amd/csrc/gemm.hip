@@ -18,6 +18,7 @@
 
 #include "formats.h"
 #include "kernels.h"
+#include "panel.h"
 
 namespace nuq {
 
@@ -322,19 +323,6 @@ struct WRaw<12> {
         hdr = *(const u32x4 *)blk;
         qs = *(const u32x4 *)(blk + 16 + (ks & 3) * 32 + part * 16);
     }
-    // The same two loads as asm, which the compiler does not track: the
-    // caller waits with wait<N>(), N = vector memory ops issued after them.
-    __device__ __forceinline__ void load_asm(const uint8_t *row, uint32_t ks, uint32_t part) {
-        const uint8_t *blk = row + (uint64_t)(ks >> 2) * 144;
-        const uint8_t *q = blk + 16 + (ks & 3) * 32 + part * 16;
-        asm volatile("global_load_dwordx4 %0, %2, off\n\tglobal_load_dwordx4 %1, %3, off"
-                     : "=&v"(hdr), "=&v"(qs) : "v"(blk), "v"(q) : "memory");
-    }
-    template <int N>
-    __device__ __forceinline__ void wait() {
-        asm volatile("s_waitcnt vmcnt(%2)" : "+v"(hdr), "+v"(qs) : "n"(N) : "memory");
-    }
-
     __device__ __forceinline__ void dequant(uint32_t ks, uint32_t part, uint32_t c, _Float16 *out) {
         if (c == 0) {
             const uint32_t p = ks & 3;
@@ -364,25 +352,6 @@ struct WRaw<14> {
     u32x4 ql, qh, sc16;
     uint32_t d16;
     float mul_lo, mul_hi;
-    // load() as asm (three unaligned 16-byte loads and one 2-byte load),
-    // untracked by the compiler: wait<N>() as for WRaw<12>
-    __device__ __forceinline__ void load_asm(const uint8_t *row, uint32_t ks, uint32_t part) {
-        const uint8_t *blk = row + (uint64_t)(ks >> 2) * 210;
-        const uint32_t h = (ks & 3) >> 1, qa = ks & 1;
-        const uint8_t *pa = blk + h * 64 + qa * 32 + 16 * part, *pb = blk + 128 + h * 32 + 16 * part;
-        asm volatile(
-            "global_load_dwordx4 %0, %4, off\n\t"
-            "global_load_dwordx4 %1, %5, off\n\t"
-            "global_load_dwordx4 %2, %6, off offset:192\n\t"
-            "global_load_ushort %3, %6, off offset:208"
-            : "=&v"(ql), "=&v"(qh), "=&v"(sc16), "=&v"(d16)
-            : "v"(pa), "v"(pb), "v"(blk)
-            : "memory");
-    }
-    template <int N>
-    __device__ __forceinline__ void wait() {
-        asm volatile("s_waitcnt vmcnt(%4)" : "+v"(ql), "+v"(qh), "+v"(sc16), "+v"(d16) : "n"(N) : "memory");
-    }
     __device__ __forceinline__ void load(const uint8_t *row, uint32_t ks, uint32_t part) {
         const uint8_t *blk = row + (uint64_t)(ks >> 2) * 210;
         const uint32_t h = (ks & 3) >> 1, qa = ks & 1;
@@ -429,22 +398,6 @@ struct WRaw<13> {
         qh = *(const u32x4 *)(blk + 16 + part * 16);
         qs = *(const u32x4 *)(blk + 48 + (ks & 3) * 32 + part * 16);
     }
-    // load() as asm, untracked by the compiler: wait<N>() as for WRaw<12>
-    __device__ __forceinline__ void load_asm(const uint8_t *row, uint32_t ks, uint32_t part) {
-        const uint8_t *blk = row + (uint64_t)(ks >> 2) * 176;
-        const uint8_t *ph = blk + 16 + part * 16, *pq = blk + 48 + (ks & 3) * 32 + part * 16;
-        asm volatile(
-            "global_load_dwordx4 %0, %3, off\n\t"
-            "global_load_dwordx4 %1, %4, off\n\t"
-            "global_load_dwordx4 %2, %5, off"
-            : "=&v"(hdr), "=&v"(qh), "=&v"(qs)
-            : "v"(blk), "v"(ph), "v"(pq)
-            : "memory");
-    }
-    template <int N>
-    __device__ __forceinline__ void wait() {
-        asm volatile("s_waitcnt vmcnt(%3)" : "+v"(hdr), "+v"(qh), "+v"(qs) : "n"(N) : "memory");
-    }
     __device__ __forceinline__ void dequant(uint32_t ks, uint32_t part, uint32_t c, _Float16 *out) {
         if (c == 0) {
             const uint32_t p = ks & 3;
@@ -487,22 +440,6 @@ struct WRaw<23> {
         q01 = *(const u32x2 *)(blk + 8 + 16 * g);
         q23 = *(const u32x2 *)(blk + 16 + 16 * g);
     }
-    // load() as asm, untracked by the compiler: wait<N>() as for WRaw<12>
-    __device__ __forceinline__ void load_asm(const uint8_t *row, uint32_t ks, uint32_t part) {
-        const uint8_t *blk = row + (uint64_t)(ks >> 2) * 136;
-        const uint8_t *pq = blk + 8 + 16 * (2 * (ks & 3) + part);
-        asm volatile(
-            "global_load_dwordx2 %0, %3, off\n\t"
-            "global_load_dwordx2 %1, %4, off\n\t"
-            "global_load_dwordx2 %2, %4, off offset:8"
-            : "=&v"(hdr), "=&v"(q01), "=&v"(q23)
-            : "v"(blk), "v"(pq)
-            : "memory");
-    }
-    template <int N>
-    __device__ __forceinline__ void wait() {
-        asm volatile("s_waitcnt vmcnt(%3)" : "+v"(hdr), "+v"(q01), "+v"(q23) : "n"(N) : "memory");
-    }
     // this thread owns group 2(ks&3) + part: chunk c = byte dword c, values
     // 4c..4c+3 (low nibbles) and 16+4c.. (high nibbles)
     __device__ __forceinline__ void dequant(uint32_t ks, uint32_t part, uint32_t c, _Float16 *out) {
@@ -542,7 +479,8 @@ struct WRaw<8> {
         qa = u32x4{a.x, a.y, a.z, a.w};
         qb = u32x4{b.x, b.y, b.z, b.w};
     }
-    // load() as asm, untracked by the compiler: wait<N>() as for WRaw<12>
+    // load() as asm, which the compiler does not track: the caller waits with
+    // wait<N>(), N = vector memory ops issued after them
     __device__ __forceinline__ void load_asm(const uint8_t *row, uint32_t ks, uint32_t part) {
         const uint8_t *blk = row + (uint64_t)(2 * ks + part) * 34;
         asm volatile(
@@ -579,17 +517,14 @@ constexpr int PF_BM = 256, PF_BN = 256, PF_GROUP_M = 4;
 #define NUQ_PF_COPY_FIRST_MASK ((1u << 8) | (1u << 13) | (1u << 14))
 #endif
 template <uint32_t ENC> struct PF_COPY_FIRST { static constexpr bool value = (NUQ_PF_COPY_FIRST_MASK >> (ENC & 31)) & 1u; };
-// With f16 activations the weight prefetch is asm loads the compiler does
-// not track, issued after the activation copies: the step's end then waits
+// With f16 activations (Q8_0) the weight prefetch is asm loads the compiler
+// does not track, issued after the activation copies: the step's end then waits
 // for the copies only and the weights keep their two-step distance (the
 // compiler's own waits fall back to vmcnt(0) behind LDS copies). A/B on one
-// box, M=4096 / M=512 TFLOP/s: Q4_K 848-861 -> 857-858 / 562-569 -> 585-589,
-// Q6_K 779-781 -> 807-809 / 577-591 -> 588-601, Q5_K 794-806 -> 844-850 /
-// 606-614 -> 630-637, IQ4_XS 850-860 -> 870-881 / 614-629 -> 652-670, Q8_0
-// 860-863 -> 880-892 / 599-616 -> 639-653.
+// box, M=4096 / M=512: 860-863 -> 880-892 / 599-616 -> 639-653 TFLOP/s.
 template <uint32_t ENC, typename XT> struct PF_ASMW {
     static constexpr bool value = sizeof(XT) == 2;
-    static constexpr int LOADS = ENC == 14 ? 4 : ENC == 12 ? 2 : 3;  // WRaw<ENC>::load_asm's instructions
+    static constexpr int LOADS = 3;  // WRaw<8>::load_asm's instructions
 };
 
 typedef __attribute__((address_space(3))) void lds_void_t;
@@ -975,19 +910,20 @@ static hipError_t launch_prefill(hipStream_t s, const uint8_t *w, uint64_t strid
     prefill_split_plan(tiles, columns, cus, scratch.work != nullptr ? scratch.tiles : 0, &full, &tail, &splits);
     const uint32_t grid = full + tail * splits;
     const size_t lds = (size_t)2 * (PF_BM + PF_BN) * LDS_PITCH * sizeof(_Float16);
-#define NUQ_PF_LAUNCH(NW_)                                                                                       \
-    if (x_f16)                                                                                                   \
-        hipLaunchKernelGGL((prefill_kernel<ENC, _Float16, NW_>), dim3(grid), dim3(64 * NW_), lds, s, w, stride,  \
-                           rows, columns, (const _Float16 *)x, in_stride, y, out_stride, tokens, full, tail,     \
-                           splits, scratch.work);                                                                \
-    else                                                                                                         \
-        hipLaunchKernelGGL((prefill_kernel<ENC, float, NW_>), dim3(grid), dim3(64 * NW_), lds, s, w, stride, rows, \
-                           columns, (const float *)x, in_stride, y, out_stride, tokens, full, tail, splits,      \
-                           scratch.work);
     // 8 waves: NW = 4 (1 wave per SIMD) measured slower on MI355X, 693 vs
-    // 753 TFLOP/s for Q4_K 17408 x 5120 at 4096 tokens
-    NUQ_PF_LAUNCH(8)
-#undef NUQ_PF_LAUNCH
+    // 753 TFLOP/s for Q4_K 17408 x 5120 at 4096 tokens. f16 activations come
+    // here for Q8_0 only (see plan_tile).
+    if constexpr (ENC == 8) {
+        if (x_f16)
+            hipLaunchKernelGGL((prefill_kernel<ENC, _Float16, 8>), dim3(grid), dim3(512), lds, s, w, stride, rows,
+                               columns, (const _Float16 *)x, in_stride, y, out_stride, tokens, full, tail, splits,
+                               scratch.work);
+    } else if (x_f16) {
+        return hipErrorInvalidValue;
+    }
+    if (!x_f16)
+        hipLaunchKernelGGL((prefill_kernel<ENC, float, 8>), dim3(grid), dim3(512), lds, s, w, stride, rows, columns,
+                           (const float *)x, in_stride, y, out_stride, tokens, full, tail, splits, scratch.work);
     if (tail != 0)
         hipLaunchKernelGGL(split_reduce_kernel, dim3(tail * (PF_BM * PF_BN / 256)), dim3(256), 0, s, scratch.work, y,
                            out_stride, rows, tokens, full, splits);
@@ -2385,12 +2321,8 @@ uint32_t split_scratch_tiles() { return 4 * compute_units(); }
 
 // Q4_K / Q5_K with up to VF_PASS_MAX tokens (K a multiple of 256) run on the
 // streamed verify tile in passes of at most 16 tokens, each pass reading the
-// weights once; more tokens, and the other encodings past 16 tokens, go to
-// the prefill tile. 17408 x 5120 Q4_K: 17 / 24 / 32 / 48 tokens 0.033 /
-// 0.034 / 0.047 / 0.070 ms in passes against 0.075-0.078 on the prefill
-// tile (and 0.108-0.126 on the 128 x 128 tile); Q6_K 5120 x 17408, whose
-// verify tile is the register form, 0.083 in passes at 17 tokens against
-// 0.078.
+// weights once (17408 x 5120 Q4_K: 17 / 24 / 32 / 48 tokens 33 / 34 / 47 /
+// 70 us): its products are exact where the other tiles round weights to f16.
 constexpr uint32_t VF_PASS_MAX = 48;
 static bool vf_passes(uint32_t encoding, uint32_t tokens, uint32_t columns) {
     return (encoding == 12 || encoding == 13) && tokens > 16 && tokens <= VF_PASS_MAX && columns % 256 == 0;
@@ -2400,70 +2332,190 @@ static uint32_t vf_pass_tokens(uint32_t tokens) {
     return (tokens + passes - 1) / passes;
 }
 
-uint64_t tile_workspace_floats(uint32_t encoding, uint32_t rows, uint32_t columns, uint32_t tokens,
-                               uint64_t in_stride, bool xs3) {
-    if (vf_passes(encoding, tokens, columns)) tokens = vf_pass_tokens(tokens);
-    if (tokens <= 16 && columns % 256 == 0) {
-        // the streamed verify tile's K ranges (Q4_K / Q5_K rows longer than
-        // 2 * MAXW blocks, or 20 for the F32 multi-token form), one F32
-        // partial per range, token and row
-        constexpr uint32_t MAXW = vd_max_waves<2>();
-        const uint32_t nblocks = columns / 256, max_kb = vd_max_kb(xs3);
-        if ((encoding != 12 && encoding != 13) || nblocks <= max_kb || rows < 16) return 0;
-        return (uint64_t)((nblocks + max_kb - 1) / max_kb) * tokens * rows;
+uint64_t verify_workspace_floats(uint32_t encoding, uint32_t rows, uint32_t columns, uint32_t tokens, bool xs3) {
+    // the streamed verify tile's K ranges (Q4_K / Q5_K rows longer than
+    // 2 * MAXW blocks, or 20 for the F32 multi-token form), one F32
+    // partial per range, token and row
+    const uint32_t nblocks = columns / 256, max_kb = vd_max_kb(xs3);
+    if ((encoding != 12 && encoding != 13) || nblocks <= max_kb || rows < 16) return 0;
+    return (uint64_t)((nblocks + max_kb - 1) / max_kb) * tokens * rows;
+}
+
+// Predicted time (us) of Q8_0 on the prefill tile with f16 activations: 3.6 us
+// a round of 256 tiles, 8.54 us a 256-column block of a round, 0.4 us per MB of
+// split partial sums. Fitted to the times from 64 to 4096 tokens on 17408 x
+// 5120, 5120 x 17408 and 4096 x 4096 (6 % rms).
+static float prefill_cost(uint32_t rows, uint32_t columns, uint32_t tokens, uint64_t max_floats) {
+    const uint32_t tiles = ((tokens + PF_BM - 1) / PF_BM) * ((rows + PF_BN - 1) / PF_BN), nb = columns / 256;
+    uint32_t full, tail, splits;
+    prefill_split_plan(tiles, columns, 256, max_floats / (PF_BM * PF_BN), &full, &tail, &splits);
+    const uint32_t r1 = (full + 255) / 256, r2 = (tail * splits + 255) / 256;
+    return 3.6f * (r1 + r2) + 8.54f * (r1 * nb + r2 * ((nb + splits - 1) / splits)) +
+           0.4f * (float)tail * splits * (PF_BM * PF_BN * 4e-6f);
+}
+
+// At most this much f16 copy of F32 activations at a time (bytes).
+constexpr uint64_t X16_BYTES = 1ull << 30;
+
+// The route of a product on the tiles, with at most max_floats of workspace.
+//  - Q4_K / Q5_K up to VF_PASS_MAX tokens keep the streamed verify tile, whose
+//    products are exact (the panel tile rounds weights to f16).
+//  - Otherwise the panel tile, from 17 tokens, and from 4 for matrices of at
+//    least 2^25 weights: Q6_K 5120 x 17408 at 4 / 16 tokens 28 / 29 us against
+//    38 / 44 on the register verify tile, 5120 x 6144 15.8 / 16 against
+//    15.8 / 18, 4096 x 4096 11-15 against 7-10 (it needs the split and its
+//    reduction there).
+//  - Q8_0 may run on the prefill tile where that is predicted faster: its raw
+//    bytes are twice the others', and the panel tile reads them once per 128 or
+//    256 tokens of every row tile through LDS (17408 x 5120 at 4096 tokens 779
+//    us against 815, at 256 tokens 84 against 98; 4096 x 4096 at 256 tokens
+//    34.6 against 28). The panel model is a little low there, so the panel has
+//    to win by 8 %.
+//  - F32 activations are rounded to f16 in one pass first (the tiles round
+//    them anyway; Q6_K 5120 x 17408 at 1999 tokens 711 us with the rounding
+//    inside the prefill tile). Without workspace for the copy (a call
+//    recorded into a graph before any was allocated) the prefill tile's own
+//    F32 form serves them.
+void plan_tile(uint32_t encoding, uint32_t rows, uint32_t columns, uint32_t tokens, uint32_t x_f16, uint64_t stride,
+               uint64_t in_stride, uint64_t max_floats, TilePlan *t) {
+    *t = TilePlan{};
+    t->chunk = tokens;
+    if (vf_passes(encoding, tokens, columns)) {
+        t->route = TilePlan::VERIFY;
+        t->floats = verify_workspace_floats(encoding, rows, columns, vf_pass_tokens(tokens), false);
+        return;
     }
-    if (tokens > 16 && (uint64_t)PF_BM * in_stride * 2 + 256 <= 0xffffffffull) {  // as launch_tile routes
-        const uint32_t cus = compute_units();
-        const uint32_t tiles = ((tokens + PF_BM - 1) / PF_BM) * ((rows + PF_BN - 1) / PF_BN);
-        uint32_t full, tail, splits;
-        prefill_split_plan(tiles, columns, cus, split_scratch_tiles(), &full, &tail, &splits);
-        return (uint64_t)tail * splits * PF_BM * PF_BN;
+    const bool small = tokens <= 16 && columns % 256 == 0;
+    const bool split_tile = encoding == 12 || encoding == 13;
+    const bool offsets32 = (uint64_t)PF_BM * in_stride * 2 + 256 <= 0xffffffffull;  // the prefill tile's copies
+    if (small) {
+        t->route = TilePlan::VERIFY;
+        t->floats = verify_workspace_floats(encoding, rows, columns, tokens, false);
+        if (split_tile || tokens < 4 || (uint64_t)rows * columns < (1ull << 25)) return;
+    } else {
+        t->route = tokens > 16 && offsets32 ? TilePlan::PREFILL : TilePlan::TILE;
     }
-    return 0;
+    // f16 rows of a chunk of the tokens, behind the split's partial tiles
+    uint32_t chunk = tokens;
+    uint64_t copy = 0;
+    if (!x_f16) {
+        chunk = (uint32_t)std::min<uint64_t>(tokens, X16_BYTES / 2 / columns);
+        if (chunk < tokens) chunk = chunk / 256 * 256;
+        copy = ((uint64_t)chunk * columns + 1) / 2;
+    }
+    const uint64_t row_stride = x_f16 ? in_stride : columns;
+    const uint64_t split_max = (uint64_t)split_scratch_tiles() * PF_BM * PF_BN;
+    const bool room = chunk != 0 && copy <= max_floats;
+    if (room && panel_plan(encoding, rows, columns, chunk, stride, row_stride, std::min(max_floats - copy, split_max),
+                           &t->panel)) {
+        const bool both = !small && t->route == TilePlan::PREFILL && encoding == 8;
+        if (!both ||
+            t->panel.cost < 0.92f * prefill_cost(rows, columns, chunk, std::min(max_floats - copy, split_max))) {
+            t->route = TilePlan::PANEL;
+            t->chunk = chunk;
+            t->copy = copy;
+            t->floats = t->panel.work_floats + copy;
+            return;
+        }
+    }
+    if (t->route != TilePlan::PREFILL) return;
+    // the prefill tile: f16 rows for Q8_0, else its F32 form
+    const bool convert = !x_f16 && room && encoding == 8 &&
+                         (uint64_t)PF_BM * columns * 2 + 256 <= 0xffffffffull;
+    t->chunk = convert ? chunk : tokens;
+    t->copy = convert ? copy : 0;
+    if (x_f16 && encoding != 8) {
+        t->route = TilePlan::TILE;  // a row stride beyond the panel tile's 32-bit offsets
+        return;
+    }
+    const uint32_t tiles = ((t->chunk + PF_BM - 1) / PF_BM) * ((rows + PF_BN - 1) / PF_BN);
+    uint32_t full, tail, splits;
+    prefill_split_plan(tiles, columns, compute_units(), std::min(max_floats - t->copy, split_max) / (PF_BM * PF_BN),
+                       &full, &tail, &splits);
+    t->floats = (uint64_t)tail * splits * PF_BM * PF_BN + t->copy;
+}
+
+static hipError_t launch_verify(hipStream_t s, uint32_t encoding, const uint8_t *w, uint64_t stride, uint32_t rows,
+                                uint32_t columns, const void *x, uint32_t x_f16, uint64_t in_stride, float *y,
+                                uint64_t out_stride, uint32_t tokens, const SplitScratch &scratch) {
+    switch (encoding) {
+    case 12: return launch_verify_enc<12>(s, w, stride, rows, columns, x, x_f16, in_stride, y, out_stride, tokens, scratch);
+    case 13: return launch_verify_enc<13>(s, w, stride, rows, columns, x, x_f16, in_stride, y, out_stride, tokens, scratch);
+    case 14: return launch_verify_enc<14>(s, w, stride, rows, columns, x, x_f16, in_stride, y, out_stride, tokens, scratch);
+    case 23: return launch_verify_enc<23>(s, w, stride, rows, columns, x, x_f16, in_stride, y, out_stride, tokens, scratch);
+    default: return launch_verify_enc<8>(s, w, stride, rows, columns, x, x_f16, in_stride, y, out_stride, tokens, scratch);
+    }
+}
+
+static hipError_t launch_prefill_any(hipStream_t s, uint32_t encoding, const uint8_t *w, uint64_t stride, uint32_t rows,
+                                     uint32_t columns, const void *x, uint32_t x_f16, uint64_t in_stride, float *y,
+                                     uint64_t out_stride, uint32_t tokens, const SplitScratch &scratch) {
+    const uint32_t cus = compute_units();
+    switch (encoding) {
+    case 12: return launch_prefill<12>(s, w, stride, rows, columns, x, x_f16, in_stride, y, out_stride, tokens, scratch, cus);
+    case 13: return launch_prefill<13>(s, w, stride, rows, columns, x, x_f16, in_stride, y, out_stride, tokens, scratch, cus);
+    case 14: return launch_prefill<14>(s, w, stride, rows, columns, x, x_f16, in_stride, y, out_stride, tokens, scratch, cus);
+    case 23: return launch_prefill<23>(s, w, stride, rows, columns, x, x_f16, in_stride, y, out_stride, tokens, scratch, cus);
+    default: return launch_prefill<8>(s, w, stride, rows, columns, x, x_f16, in_stride, y, out_stride, tokens, scratch, cus);
+    }
 }
 
 hipError_t launch_tile(hipStream_t s, uint32_t encoding, const uint8_t *w, uint64_t stride, uint32_t rows,
                        uint32_t columns, const void *x, uint32_t x_f16, uint64_t in_stride, float *y,
-                       uint64_t out_stride, uint32_t tokens, const SplitScratch &scratch) {
-    if (vf_passes(encoding, tokens, columns)) {
+                       uint64_t out_stride, uint32_t tokens, const TilePlan &plan, const SplitScratch &scratch) {
+    if (plan.route == TilePlan::VERIFY) {
+        // passes of at most 16 tokens, each reading the weights once
         const uint32_t chunk = vf_pass_tokens(tokens);
         const size_t xe = x_f16 ? 2 : 4;
         for (uint32_t t0 = 0; t0 < tokens; t0 += chunk) {
-            const hipError_t e = launch_tile(s, encoding, w, stride, rows, columns,
-                                             (const uint8_t *)x + (uint64_t)t0 * in_stride * xe, x_f16, in_stride,
-                                             y + (uint64_t)t0 * out_stride, out_stride, std::min(chunk, tokens - t0),
-                                             scratch);
+            const hipError_t e = launch_verify(s, encoding, w, stride, rows, columns,
+                                               (const uint8_t *)x + (uint64_t)t0 * in_stride * xe, x_f16, in_stride,
+                                               y + (uint64_t)t0 * out_stride, out_stride, std::min(chunk, tokens - t0),
+                                               scratch);
             if (e != hipSuccess) return e;
         }
         return hipSuccess;
     }
-    if (tokens <= 16 && columns % 256 == 0) {
+    if (plan.route == TilePlan::TILE || (plan.route == TilePlan::PREFILL && plan.copy == 0)) {
+        if (plan.route == TilePlan::PREFILL)
+            return launch_prefill_any(s, encoding, w, stride, rows, columns, x, x_f16, in_stride, y, out_stride, tokens,
+                                      scratch);
         switch (encoding) {
-        case 12: return launch_verify_enc<12>(s, w, stride, rows, columns, x, x_f16, in_stride, y, out_stride, tokens, scratch);
-        case 13: return launch_verify_enc<13>(s, w, stride, rows, columns, x, x_f16, in_stride, y, out_stride, tokens, scratch);
-        case 14: return launch_verify_enc<14>(s, w, stride, rows, columns, x, x_f16, in_stride, y, out_stride, tokens, scratch);
-        case 23: return launch_verify_enc<23>(s, w, stride, rows, columns, x, x_f16, in_stride, y, out_stride, tokens, scratch);
-        default: return launch_verify_enc<8>(s, w, stride, rows, columns, x, x_f16, in_stride, y, out_stride, tokens, scratch);
+        case 12: return launch_tile_enc<12>(s, w, stride, rows, columns, x, x_f16, in_stride, y, out_stride, tokens);
+        case 13: return launch_tile_enc<13>(s, w, stride, rows, columns, x, x_f16, in_stride, y, out_stride, tokens);
+        case 14: return launch_tile_enc<14>(s, w, stride, rows, columns, x, x_f16, in_stride, y, out_stride, tokens);
+        case 23: return launch_tile_enc<23>(s, w, stride, rows, columns, x, x_f16, in_stride, y, out_stride, tokens);
+        default: return launch_tile_enc<8>(s, w, stride, rows, columns, x, x_f16, in_stride, y, out_stride, tokens);
         }
     }
-    // (the prefill tile's activation copies use 32-bit offsets within a tile)
-    if (tokens > 16 && (uint64_t)PF_BM * in_stride * 2 + 256 <= 0xffffffffull) {
-        const uint32_t cus = compute_units();
-        switch (encoding) {
-        case 12: return launch_prefill<12>(s, w, stride, rows, columns, x, x_f16, in_stride, y, out_stride, tokens, scratch, cus);
-        case 13: return launch_prefill<13>(s, w, stride, rows, columns, x, x_f16, in_stride, y, out_stride, tokens, scratch, cus);
-        case 14: return launch_prefill<14>(s, w, stride, rows, columns, x, x_f16, in_stride, y, out_stride, tokens, scratch, cus);
-        case 23: return launch_prefill<23>(s, w, stride, rows, columns, x, x_f16, in_stride, y, out_stride, tokens, scratch, cus);
-        default: return launch_prefill<8>(s, w, stride, rows, columns, x, x_f16, in_stride, y, out_stride, tokens, scratch, cus);
+    // f16 activations, or f16 copies of F32 ones in the workspace, chunk by chunk
+    const uint64_t split_floats = plan.floats - plan.copy;
+    _Float16 *const copy = (_Float16 *)(scratch.work + split_floats);
+    for (uint32_t t0 = 0; t0 < tokens; t0 += plan.chunk) {
+        const uint32_t n = std::min(plan.chunk, tokens - t0);
+        const _Float16 *xc = (const _Float16 *)x + (uint64_t)t0 * in_stride;
+        uint64_t xs = in_stride;
+        if (plan.copy != 0) {
+            const hipError_t e = launch_to_f16(s, (const float *)x + (uint64_t)t0 * in_stride, in_stride, columns, n, copy);
+            if (e != hipSuccess) return e;
+            xc = copy;
+            xs = columns;
         }
+        float *yc = y + (uint64_t)t0 * out_stride;
+        hipError_t e;
+        if (plan.route == TilePlan::PREFILL) {
+            const SplitScratch partials{scratch.work, (uint32_t)(split_floats / (PF_BM * PF_BN))};
+            e = launch_prefill_any(s, encoding, w, stride, rows, columns, xc, 1, xs, yc, out_stride, n, partials);
+        } else {
+            PanelPlan p = plan.panel;
+            if (n != plan.chunk &&
+                !panel_plan(encoding, rows, columns, n, stride, xs, split_floats, &p))  // a shorter last chunk
+                return hipErrorInvalidValue;
+            e = launch_panel(s, encoding, {w, stride, rows, columns, xc, xs, yc, out_stride, n}, p, scratch.work);
+        }
+        if (e != hipSuccess) return e;
     }
-    switch (encoding) {
-    case 12: return launch_tile_enc<12>(s, w, stride, rows, columns, x, x_f16, in_stride, y, out_stride, tokens);
-    case 13: return launch_tile_enc<13>(s, w, stride, rows, columns, x, x_f16, in_stride, y, out_stride, tokens);
-    case 14: return launch_tile_enc<14>(s, w, stride, rows, columns, x, x_f16, in_stride, y, out_stride, tokens);
-    case 23: return launch_tile_enc<23>(s, w, stride, rows, columns, x, x_f16, in_stride, y, out_stride, tokens);
-    default: return launch_tile_enc<8>(s, w, stride, rows, columns, x, x_f16, in_stride, y, out_stride, tokens);
-    }
+    return hipSuccess;
 }
 
 }  // namespace nuq

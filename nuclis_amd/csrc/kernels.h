@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "panel.h"
+
 namespace nuq {
 
 struct SegmentDesc {
@@ -73,9 +75,20 @@ hipError_t launch_penalize(hipStream_t s, float *logits, uint32_t count, const u
                            float presence);
 hipError_t launch_topk(hipStream_t s, const float *logits, uint32_t count, uint32_t k, float temperature,
                        uint64_t *scratch, float *values, uint32_t *indices, float *sums, uint32_t *flags);
+// How a product runs on the tiles (plan_tile): the route, its panel plan, the
+// tokens served per chunk, the floats of the f16 copy of F32 activations and
+// the workspace it uses in all (split partials, then the copy).
+struct TilePlan {
+    enum Route { VERIFY, PANEL, PREFILL, TILE } route;
+    PanelPlan panel;
+    uint32_t chunk;
+    uint64_t copy, floats;
+};
+void plan_tile(uint32_t encoding, uint32_t rows, uint32_t columns, uint32_t tokens, uint32_t x_f16, uint64_t stride,
+               uint64_t in_stride, uint64_t max_floats, TilePlan *plan);
 hipError_t launch_tile(hipStream_t s, uint32_t encoding, const uint8_t *w, uint64_t stride, uint32_t rows,
                        uint32_t columns, const void *x, uint32_t x_f16, uint64_t in_stride, float *y,
-                       uint64_t out_stride, uint32_t tokens, const SplitScratch &scratch);
+                       uint64_t out_stride, uint32_t tokens, const TilePlan &plan, const SplitScratch &scratch);
 uint32_t split_scratch_tiles();
 // Adds `ranges` K-range partial outputs ws[(k * tokens + t) * rows + r] in
 // range order into y[t * out_stride + r].
@@ -95,10 +108,8 @@ bool launch_rows_q4k_f16(hipStream_t s, const uint8_t *w, uint64_t stride, uint3
 hipError_t launch_rows_mfma(hipStream_t s, uint32_t encoding, const uint8_t *w, uint64_t stride, uint32_t rows,
                             uint32_t columns, const float *x, uint64_t in_stride, float *y, uint64_t out_stride,
                             uint32_t tokens, const SplitScratch &scratch, bool *taken);
-// F32 workspace the tile route of this call would use (verify K ranges or
-// prefill split partials); 0 when it needs none. A smaller workspace makes
-// the route fall back (fewer splits, or the register verify tile).
-uint64_t tile_workspace_floats(uint32_t encoding, uint32_t rows, uint32_t columns, uint32_t tokens,
-                               uint64_t in_stride, bool xs3 = false);
+// F32 workspace of the streamed verify tile's K ranges; 0 when it needs
+// none. With less, the register verify tile serves the call.
+uint64_t verify_workspace_floats(uint32_t encoding, uint32_t rows, uint32_t columns, uint32_t tokens, bool xs3);
 
 }  // namespace nuq
