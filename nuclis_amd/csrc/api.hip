@@ -616,7 +616,19 @@ static int segments_impl(nuq_context *ctx, const nuq_segment *segments, uint32_t
         return fail(ctx, NUQ_INVALID_SHAPE,
                     "SiLU pair of %llu rows exceeds the allocation-free scratch (at most %llu rows)",
                     (unsigned long long)segments[0].matrix.rows, (unsigned long long)fixed_floats);
-    // A large SiLU pair streams faster as decode GEMVs (gate into the output,
+    bool same = !ctx->generic_only;
+    for (uint32_t i = 1; i < count && same; ++i)
+        same = segments[i].matrix.encoding == segments[0].matrix.encoding && strides[i] == strides[0];
+    // A large SiLU pair of one encoding is one launch of the decode GEMV with
+    // the epilogue on its own sums.
+    if (same && mode == NUQ_SEGMENT_SILU_MUL_PAIR && segments[0].matrix.rows >= PAIR_SPLIT_ROWS) {
+        const nuq_matrix &g = segments[0].matrix;
+        const hipError_t he = nuq::launch_gemv_dma_pair(ctx->stream, g.encoding, (const uint8_t *)g.bytes,
+                                                        (const uint8_t *)segments[1].matrix.bytes, strides[0],
+                                                        (uint32_t)g.rows, (uint32_t)columns, x, segments[0].output);
+        if (he != hipErrorInvalidValue) return hip_check(ctx, he, "silu pair launch");
+    }
+    // Other large pairs stream faster as decode GEMVs (gate into the output,
     // up into a workspace) and the elementwise epilogue than as one merged
     // row-per-wave pass.
     const bool pair_big = mode == NUQ_SEGMENT_SILU_MUL_PAIR && !ctx->generic_only &&
@@ -625,10 +637,7 @@ static int segments_impl(nuq_context *ctx, const nuq_segment *segments, uint32_t
     float *up_buffer = fixed ? fixed : ctx->split.work;
     // Segments of one encoding and row stride (q/k/v, gate/up) run as one
     // launch of the decode GEMV, each matrix on its share of the workgroups.
-    bool same = !ctx->generic_only && (mode == NUQ_SEGMENT_PLAIN || pair_split);
-    for (uint32_t i = 1; i < count && same; ++i)
-        same = segments[i].matrix.encoding == segments[0].matrix.encoding && strides[i] == strides[0];
-    if (same) {
+    if (same && (mode == NUQ_SEGMENT_PLAIN || pair_split)) {
         const uint8_t *ws[4];
         uint32_t rs[4];
         float *ys[4];

@@ -805,6 +805,9 @@ __device__ __forceinline__ float group_sum(float v) {
     return v;
 }
 
+// silu as cpu/vector.zig:178-181 and the segments kernel: -inf maps to -0
+__device__ __forceinline__ float silu_f32(float g) { return g == -INFINITY ? -0.f : g / (1.f + expf(-g)); }
+
 // Workgroup size cap of the DMA kernel: 16 waves, except Q6_K, whose lanes
 // hold more bytes per block (the alignment shifts) and so take 12 waves,
 // keeping its registers (up to 170) clear of spills.
@@ -816,7 +819,9 @@ constexpr int gd_threads() { return ENC == 14 ? 768 : GI_WG_THREADS; }
 // before their explicit waits, and a branch merging two forms made the
 // compiler copy them early).
 // WX: every wave quantises its own blocks' x slices (one wave set).
-template <uint32_t ENC, int SLOTS, int D, bool TWO = false, bool WX = false>
+// PAIR: silu(w x) * (segs.w[1] x), both matrices' rows in one workgroup (a
+// template parameter: the row steps' extra selects cost the plain form 2 %).
+template <uint32_t ENC, int SLOTS, int D, bool TWO = false, bool WX = false, bool PAIR = false>
 __global__ void __launch_bounds__(gd_threads<ENC>()) gemv_dma_kernel(const uint8_t *__restrict__ w, uint64_t stride,
                                                                       uint32_t rows, uint32_t nblocks,
                                                                       uint32_t rows_per_wg, uint32_t set_waves,
@@ -884,6 +889,10 @@ __global__ void __launch_bounds__(gd_threads<ENC>()) gemv_dma_kernel(const uint8
     const uint32_t shift = direct ? 16 * j : 16 * j - 32;
     const uint32_t row_begin = blk * rows_per_wg;
     const uint32_t row_end = min(row_begin + rows_per_wg, rows);
+    // A pair's steps: `half` of the gate's rows, then as many of the up
+    // matrix's, whose partial sums follow the gate's.
+    const uint32_t prows = PAIR ? 2 * rows_per_wg : rows_per_wg;
+    const uint32_t half = (row_end - row_begin + GROUPS - 1) / GROUPS, tsteps = PAIR ? 2 * half : half;
     const uint32_t b = SLOTS * kw + slot;
     const bool live = b < nblocks;
     const uint32_t first = row_begin + set * GROUPS;
@@ -916,6 +925,20 @@ __global__ void __launch_bounds__(gd_threads<ENC>()) gemv_dma_kernel(const uint8
     const uint8_t *wg_base = w + (uint64_t)row_begin * stride;
     const uint32_t stride32 = (uint32_t)stride;
     const uint32_t first_local = first - row_begin, last_local = row_end - 1 - row_begin;
+    const uint8_t *up_base = (PAIR ? segs.w[1] : w) + (uint64_t)row_begin * stride;
+    // row step C_ (uniform) into a ring slot
+#define NUQ_GD_DMA2(SLOT_, C_)                                                                                \
+    {                                                                                                         \
+        const bool up_ = PAIR && (C_) >= half;                                                                        \
+        const uint8_t *base_ = up_ ? up_base : wg_base;                                                       \
+        const uint32_t cc_ = up_ ? (C_) - half : (C_);                                                        \
+        _Pragma("unroll") for (uint32_t n = 0; n < GD_DMA_INSTRS; ++n) {                                      \
+            const uint32_t lrow_ = min(cc_ * GROUPS + dq[n], last_local);                                     \
+            __builtin_amdgcn_global_load_lds((gd_global_void_t *)(base_ + (lrow_ * stride32 + doff[n])),      \
+                                             (gd_lds_void_t *)(NUQ_GD_RING(SLOT_) + n * 1024), 16, 0, 2);     \
+        }                                                                                                     \
+    }
+    const uint32_t set_s = PAIR ? __builtin_amdgcn_readfirstlane(set) : set;
 
     const uint32_t t0 = threadIdx.x;
     if constexpr (WX) {
@@ -958,7 +981,10 @@ __global__ void __launch_bounds__(gd_threads<ENC>()) gemv_dma_kernel(const uint8
     // (5120 x 17408: 16.2 -> 15.6 us for Q4_K, 19.5 -> 18.8 us for Q5_K).
     if constexpr (two_rounds) __builtin_amdgcn_s_barrier();
 #pragma unroll
-    for (int d = 0; d < D; ++d) NUQ_GD_DMA(d, (uint32_t)d)
+    for (int d = 0; d < D; ++d) {
+        if constexpr (PAIR) NUQ_GD_DMA2(d, set_s + (uint32_t)d * sets)
+        else NUQ_GD_DMA(d, (uint32_t)d)
+    }
 
     // The slice image goes to LDS through asm and the barrier carries no
     // fence, so the copies in flight keep flying while x is quantised.
@@ -977,7 +1003,7 @@ __global__ void __launch_bounds__(gd_threads<ENC>()) gemv_dma_kernel(const uint8
         quantize_half_slice<true>(xh, t & 1, slices + (t >> 1) * SLICE_WORDS);
     }
     // the row-step counters of the K ranges (D * sets steps are assigned statically)
-    if (t0 < set_waves) ((uint32_t *)(partial + rows_per_wg * set_waves + nwaves))[t0] = D * sets;
+    if (t0 < set_waves) ((uint32_t *)(partial + prows * set_waves + nwaves))[t0] = D * sets;
     asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory");
     __builtin_amdgcn_s_barrier();
     }
@@ -998,7 +1024,7 @@ __global__ void __launch_bounds__(gd_threads<ENC>()) gemv_dma_kernel(const uint8
     // wave-uniform: does any slice this wave reads hold a non-finite value
     const bool nonfinite = __ballot((xa.pos | xa.neg | xb.pos | xb.neg) != 0u) != 0;
     const uint32_t role = g * ROW_CHUNKS * 16 + slot * BYTES;
-    const uint32_t spare = rows_per_wg * set_waves + wv;  // one spare partial per wave
+    const uint32_t spare = prows * set_waves + wv;  // one spare partial per wave
 
     // Each ring slot holds one step. As soon as a slot's bytes are in
     // registers the slot is refilled with the wave's next step, before the
@@ -1017,31 +1043,26 @@ __global__ void __launch_bounds__(gd_threads<ENC>()) gemv_dma_kernel(const uint8
         partial[row < row_end ? (row - row_begin) * set_waves + kw : spare] = v;                            \
     }
     if constexpr (!WX) {
-#define NUQ_GD_DMA2(SLOT_, C_)                                                                                \
-    _Pragma("unroll") for (uint32_t n = 0; n < GD_DMA_INSTRS; ++n) {                                          \
-        const uint32_t lrow_ = min((C_) * GROUPS + dq[n], last_local);                                        \
-        __builtin_amdgcn_global_load_lds((gd_global_void_t *)(wg_base + (lrow_ * stride32 + doff[n])),        \
-                                         (gd_lds_void_t *)(NUQ_GD_RING(SLOT_) + n * 1024), 16, 0, 2);         \
-    }
 #define NUQ_GD_COMPUTE2(SLOT_, C_, VM_, REFILL_)                                                            \
     {                                                                                                       \
         GdEnc<ENC> e_;                                                                                      \
         e_.template read<VM_>(NUQ_GD_RING(SLOT_) + role, j);                                                \
         REFILL_                                                                                             \
         const float v = group_sum<4 * SLOTS>(live ? e_.dot(xa, xb, j, shift, direct) : 0.f);                \
-        const uint32_t row = row_begin + (C_) * GROUPS + g;                                                 \
-        partial[row < row_end ? (row - row_begin) * set_waves + kw : spare] = v;                            \
+        const bool up_ = PAIR && (C_) >= half;                                                              \
+        const uint32_t lrow_ = (up_ ? (C_) - half : (C_)) * GROUPS + g;                                     \
+        const uint32_t prow_ = up_ ? lrow_ + rows_per_wg : lrow_;                                           \
+        partial[lrow_ <= last_local ? prow_ * set_waves + kw : spare] = v;                                  \
     }
         // Waves of one K range (one per wave set) claim row steps from a
         // shared LDS counter, so waves that start late take fewer steps.
-        const uint32_t tsteps = (row_end - row_begin + GROUPS - 1) / GROUPS;
         const uint32_t claim_addr =
-            lds_u8_addr((const uint8_t *)(partial + rows_per_wg * set_waves + nwaves + kw));
+            lds_u8_addr((const uint8_t *)(partial + prows * set_waves + nwaves + kw));
         uint32_t sid[D];
         bool claiming = true;
 #pragma unroll
         for (int d = 0; d < D; ++d) {
-            sid[d] = set + d * sets;
+            sid[d] = set_s + d * sets;
             if (sid[d] >= tsteps) claiming = false;
         }
         while (claiming) {
@@ -1066,7 +1087,6 @@ __global__ void __launch_bounds__(gd_threads<ENC>()) gemv_dma_kernel(const uint8
         for (int d = 0; d < D; ++d)
             if (sid[d] < tsteps) NUQ_GD_COMPUTE2(d, sid[d], 0, )
 #undef NUQ_GD_COMPUTE2
-#undef NUQ_GD_DMA2
     } else {  // one wave set: each K range has one wave, steps in order
     uint32_t i = 0;
     for (; i + 2 * D <= nsteps; i += D) {
@@ -1085,6 +1105,7 @@ __global__ void __launch_bounds__(gd_threads<ENC>()) gemv_dma_kernel(const uint8
     }
 #undef NUQ_GD_COMPUTE
 #undef NUQ_GD_DMA
+#undef NUQ_GD_DMA2
 #undef NUQ_GD_RING
     // Copies issued for steps past the range (when nsteps < D) must land
     // before the workgroup ends.
@@ -1093,11 +1114,17 @@ __global__ void __launch_bounds__(gd_threads<ENC>()) gemv_dma_kernel(const uint8
     // read by some live lane, so their OR is "x holds a non-finite value".
     if (lane == 0) partial[spare] = nonfinite ? 1.f : 0.f;
     __syncthreads();
-    const bool any_nonfinite = __ballot(partial[rows_per_wg * set_waves + lane % nwaves] != 0.f) != 0;
+    const bool any_nonfinite = __ballot(partial[prows * set_waves + lane % nwaves] != 0.f) != 0;
     for (uint32_t r = threadIdx.x; r < row_end - row_begin; r += blockDim.x) {
         float t = 0.f;
         for (uint32_t k = 0; k < set_waves; ++k) t += partial[r * set_waves + k];
         if (any_nonfinite) t += nonfinite_row(ENC, w + (uint64_t)(row_begin + r) * stride, BYTES, slices, nslices);
+        if constexpr (PAIR) {
+            float u = 0.f;
+            for (uint32_t k = 0; k < set_waves; ++k) u += partial[(rows_per_wg + r) * set_waves + k];
+            if (any_nonfinite) u += nonfinite_row(ENC, up_base + (uint64_t)r * stride, BYTES, slices, nslices);
+            t = silu_f32(t) * u;
+        }
         y[row_begin + r] = t;
     }
 }
@@ -1222,6 +1249,40 @@ static hipError_t launch_dma_segments(hipStream_t s, uint32_t count, const uint8
     return hipGetLastError();
 }
 
+// silu(gate x) * (up x): one workgroup per CU streams its rows of both
+// matrices and applies the epilogue to its own sums, so the up matrix's product
+// never leaves the CU and the elementwise launch (4-5 us on MI355X) goes away.
+// Row sums are those of launch_dma.
+template <uint32_t ENC, int SLOTS, int D>
+static hipError_t launch_dma_pair(hipStream_t s, const uint8_t *gate, const uint8_t *up, uint64_t stride,
+                                  uint32_t rows, uint32_t nblocks, const float *x, float *y) {
+    constexpr uint32_t cus = 256;
+    const uint32_t set_waves = (nblocks + SLOTS - 1) / SLOTS, step_rows = 64 / (4 * SLOTS);
+    if (rows == 0 || set_waves > (uint32_t)gd_threads<ENC>() / 64) return hipErrorInvalidValue;
+    const uint32_t rpw = (rows + cus - 1) / cus;
+    if ((uint64_t)rpw * stride > 0xffffffffull) return hipErrorInvalidValue;  // 32-bit copy offsets
+    uint32_t sets = (gd_threads<ENC>() / 64) / set_waves;
+    sets = std::min(sets, std::max(1u, 2 * rpw / (2 * step_rows)));  // two steps a wave at least, as in launch_dma
+    auto lds_for = [&](uint32_t st) {
+        const size_t wv = (size_t)set_waves * st;
+        return wv * D * GdEnc<ENC>::INSTRS * 1024 + (size_t)nblocks * 8 * SLICE_WORDS * 4 +
+               ((size_t)2 * rpw * set_waves + wv + set_waves) * 4;
+    };
+    while (sets > 1 && lds_for(sets) > 160 * 1024) --sets;
+    const size_t lds = lds_for(sets);
+    if (lds > 160 * 1024) return hipErrorInvalidValue;
+    GdSegments segs{};
+    segs.w[1] = up;
+    const dim3 grid((rows + rpw - 1) / rpw), block(64 * set_waves * sets);
+    if (2 * nblocks * 8 > 64 * set_waves * sets)
+        hipLaunchKernelGGL((gemv_dma_kernel<ENC, SLOTS, D, true, false, true>), grid, block, lds, s, gate, stride, rows, nblocks,
+                           rpw, set_waves, x, y, 0u, segs);
+    else
+        hipLaunchKernelGGL((gemv_dma_kernel<ENC, SLOTS, D, false, false, true>), grid, block, lds, s, gate, stride, rows, nblocks,
+                           rpw, set_waves, x, y, 0u, segs);
+    return hipGetLastError();
+}
+
 static inline uint32_t cdiv(uint64_t a, uint64_t b) { return (uint32_t)((a + b - 1) / b); }
 
 template <int R, int SLOTS, int D>
@@ -1333,6 +1394,24 @@ hipError_t launch_gemv_dma_segments(hipStream_t s, uint32_t encoding, uint32_t c
     return hipErrorInvalidValue;
 }
 
+hipError_t launch_gemv_dma_pair(hipStream_t s, uint32_t encoding, const uint8_t *gate, const uint8_t *up,
+                                uint64_t stride, uint32_t rows, uint32_t columns, const float *x, float *y) {
+    const uint32_t nblocks = columns / 256;
+    if (columns % 256 != 0 || cdiv(nblocks, 8) > GI_MAX_SET_WAVES) return hipErrorInvalidValue;
+    const bool four = cdiv(nblocks, 4) <= GI_MAX_SET_WAVES;
+#define NUQ_GD_PAIR(E_) \
+    return four ? launch_dma_pair<E_, 4, 2>(s, gate, up, stride, rows, nblocks, x, y) \
+                : launch_dma_pair<E_, 8, 2>(s, gate, up, stride, rows, nblocks, x, y);
+    if (encoding == 12) NUQ_GD_PAIR(12)
+    if (encoding == 13) NUQ_GD_PAIR(13)
+    if (encoding == 8) NUQ_GD_PAIR(8)
+    if (encoding == 23 && nblocks % 2 == 0) NUQ_GD_PAIR(23)
+#undef NUQ_GD_PAIR
+    // the row's last copy must end with the row (launch_gemv_dma)
+    if (encoding == 14 && nblocks * 210u % 16 == 0)
+        return launch_dma_pair<14, 8, 2>(s, gate, up, stride, rows, nblocks, x, y);
+    return hipErrorInvalidValue;
+}
 
 // ---------------------------------------------------------------------------
 // Register-dequant multi-token GEMV (matvecRows form, backends/metal/kernels/

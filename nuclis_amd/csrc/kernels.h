@@ -53,6 +53,10 @@ struct GdSegments {
 hipError_t launch_gemv_dma_segments(hipStream_t s, uint32_t encoding, uint32_t count, const uint8_t *const *w,
                                     uint64_t stride, const uint32_t *rows, uint32_t columns, const float *x,
                                     float *const *y);
+// silu(gate x) * (up x) in one launch of the DMA GEMV; hipErrorInvalidValue
+// when the shape does not fit it.
+hipError_t launch_gemv_dma_pair(hipStream_t s, uint32_t encoding, const uint8_t *gate, const uint8_t *up,
+                                uint64_t stride, uint32_t rows, uint32_t columns, const float *x, float *y);
 hipError_t launch_gemv_dma(hipStream_t s, uint32_t encoding, const uint8_t *w, uint64_t stride, uint32_t rows,
                            uint32_t columns, const float *x, float *y);
 hipError_t launch_generic(hipStream_t s, uint32_t encoding, const uint8_t *w, uint64_t stride, uint32_t rows,

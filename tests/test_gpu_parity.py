@@ -453,6 +453,32 @@ def test_silu_pair_large_runs_as_two_gemvs(backend, rows):
 
 
 @pytest.mark.parametrize("encoding,columns,rows", [
+    (8, 512, 4096), (8, 17408, 4112), (12, 256, 4112), (12, 17408, 4096), (13, 5120, 4368), (14, 2048, 4352),
+    (14, 5120, 4096), (23, 512, 8208), (23, 4096, 4096),
+])
+def test_silu_pair_equals_its_gemvs(backend, encoding, columns, rows):
+    """The one-launch pair adds each row's sums as that matrix's own matvec
+    does, so it equals the epilogue over the two products to F32 rounding of
+    the epilogue; ragged row ranges, one to three wave sets, long rows."""
+    import torch
+    w = [to_gpu(quantized(encoding, rows, columns, 90 + i)) for i in range(2)]
+    mg_, mu_ = (nq.Matrix(encoding, rows, columns, t) for t in w)
+    for x in (gaussian(92, columns), np.where(np.arange(columns) == 77, np.float32(np.inf), gaussian(92, columns))):
+        xg = to_gpu(x.astype(np.float32))
+        out, g, u = (torch.full((rows,), np.nan, device="cuda") for _ in range(3))
+        backend.matvec_segments([(mg_, out), (mu_, out)], xg, nq.SEGMENT_SILU_MUL_PAIR)
+        backend.matvec(mg_, xg, g)
+        backend.matvec(mu_, xg, u)
+        backend.sync()
+        g, u = g.double(), u.double()
+        want = torch.where(g == -np.inf, -0.0, g / (1 + torch.exp(-g))) * u
+        assert torch.equal(torch.isnan(out), torch.isnan(want))
+        ok = torch.isfinite(want) & (want.abs() < 1e38)
+        # expf, the quotient and the product round once or twice each
+        assert ((out.double() - want)[ok].abs() <= 2e-6 * want[ok].abs() + 1e-37).all()
+
+
+@pytest.mark.parametrize("encoding,columns,rows", [
     (12, 5120, (6144, 1024, 1024)),   # config-3 q/k/v
     (12, 5120, (17408,)),
     (12, 17408, (512, 16, 1040, 2048)),
