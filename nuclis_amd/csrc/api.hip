@@ -619,16 +619,20 @@ static int segments_impl(nuq_context *ctx, const nuq_segment *segments, uint32_t
     bool same = !ctx->generic_only;
     for (uint32_t i = 1; i < count && same; ++i)
         same = segments[i].matrix.encoding == segments[0].matrix.encoding && strides[i] == strides[0];
-    // A large SiLU pair of one encoding is one launch of the decode GEMV with
-    // the epilogue on its own sums.
-    if (same && mode == NUQ_SEGMENT_SILU_MUL_PAIR && segments[0].matrix.rows >= PAIR_SPLIT_ROWS) {
+    // A SiLU pair of one encoding is one launch of the decode GEMV with the
+    // epilogue on its own sums, at any row count: 1024 x 5120 / 2048 x 8192
+    // take 7.2 / 7.3-9 us on MI355X, on the merged row kernel below 10 / 14 us
+    // (Q4_K, Q6_K), 12 / 17 (Q8_0) and, without a row kernel of their own,
+    // 197 / 364 (Q5_K) and 120 / 219 (IQ4_XS).
+    if (same && mode == NUQ_SEGMENT_SILU_MUL_PAIR) {
         const nuq_matrix &g = segments[0].matrix;
         const hipError_t he = nuq::launch_gemv_dma_pair(ctx->stream, g.encoding, (const uint8_t *)g.bytes,
                                                         (const uint8_t *)segments[1].matrix.bytes, strides[0],
                                                         (uint32_t)g.rows, (uint32_t)columns, x, segments[0].output);
         if (he != hipErrorInvalidValue) return hip_check(ctx, he, "silu pair launch");
     }
-    // Other large pairs stream faster as decode GEMVs (gate into the output,
+    // Other large pairs (mixed encodings, Q6_K rows that end mid-chunk) stream
+    // faster as decode GEMVs (gate into the output,
     // up into a workspace) and the elementwise epilogue than as one merged
     // row-per-wave pass.
     const bool pair_big = mode == NUQ_SEGMENT_SILU_MUL_PAIR && !ctx->generic_only &&

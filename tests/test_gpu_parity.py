@@ -455,6 +455,7 @@ def test_silu_pair_large_runs_as_two_gemvs(backend, rows):
 @pytest.mark.parametrize("encoding,columns,rows", [
     (8, 512, 4096), (8, 17408, 4112), (12, 256, 4112), (12, 17408, 4096), (13, 5120, 4368), (14, 2048, 4352),
     (14, 5120, 4096), (23, 512, 8208), (23, 4096, 4096),
+    (8, 4096, 2064), (12, 5120, 16), (13, 2048, 1024), (14, 2048, 272), (23, 512, 48),
 ])
 def test_silu_pair_equals_its_gemvs(backend, encoding, columns, rows):
     """The one-launch pair adds each row's sums as that matrix's own matvec
