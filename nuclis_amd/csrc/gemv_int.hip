@@ -808,6 +808,31 @@ __device__ __forceinline__ float group_sum(float v) {
 // silu as cpu/vector.zig:178-181 and the segments kernel: -inf maps to -0
 __device__ __forceinline__ float silu_f32(float g) { return g == -INFINITY ? -0.f : g / (1.f + expf(-g)); }
 
+// acc + the dot of values 16 s .. 16 s + 15 of a Q6_K block (one scale; 16 ql
+// and 16 qh bytes) with x, each weight in the CPU decoder's two F32 products.
+__device__ __forceinline__ float q6k_dot16(const uint8_t *blk, uint32_t s, const float *__restrict__ x, float acc) {
+    const uint32_t half = s >> 3, quarter = (s & 7) >> 1, col = 16 * (s & 1);
+    const uint8_t *pl = blk + half * 64 + (quarter & 1) * 32 + col, *ph = blk + 128 + half * 32 + col;
+    uint32_t l[4], h[4];
+    float4 xv[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        l[k] = load_u32_unaligned(pl + 4 * k);
+        h[k] = load_u32_unaligned(ph + 4 * k);
+        xv[k] = ((const float4 *)x)[k];
+    }
+    const float mul = half_bits(load_u16_bytes(blk + 208)) * (float)(int8_t)blk[192 + s];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const uint32_t u = ((l[k] >> (4 * (quarter >> 1))) & 0x0f0f0f0fu) | (((h[k] >> (2 * quarter)) & 0x03030303u) << 4);
+        acc = fmaf(mul * (float)((int)(u & 0xffu) - 32), xv[k].x, acc);
+        acc = fmaf(mul * (float)((int)((u >> 8) & 0xffu) - 32), xv[k].y, acc);
+        acc = fmaf(mul * (float)((int)((u >> 16) & 0xffu) - 32), xv[k].z, acc);
+        acc = fmaf(mul * (float)((int)(u >> 24) - 32), xv[k].w, acc);
+    }
+    return acc;
+}
+
 // Workgroup size cap of the DMA kernel: 16 waves, except Q6_K, whose lanes
 // hold more bytes per block (the alignment shifts) and so take 12 waves,
 // keeping its registers (up to 170) clear of spills.
@@ -850,11 +875,15 @@ __global__ void __launch_bounds__(gd_threads<ENC>()) gemv_dma_kernel(const uint8
     if (tail && blockIdx.x == gridDim.x - 1) {
         // The matrix's last row (rows is the count without it), when a row
         // ends mid-chunk: its last copy would read past the weights, so this
-        // extra workgroup decodes it exactly against F32 x instead.
+        // extra workgroup decodes it exactly against F32 x instead, 16 values
+        // of one scale per thread and step with all their loads at once
+        // (value by value, a chain of byte loads, this row alone took longer
+        // than the others of a small matrix: 1024 x 5120 9.4 us in all).
         const uint8_t *rowp = w + (uint64_t)rows * stride;
         float acc = 0.f;
-        for (uint32_t c = threadIdx.x; c < nblocks * 256; c += blockDim.x)
-            acc = fmaf(decode_value(ENC, rowp + (uint64_t)(c / 256) * GdEnc<ENC>::BYTES, c % 256), x[c], acc);
+        if constexpr (ENC == 14)
+            for (uint32_t c = threadIdx.x; c < nblocks * 16; c += blockDim.x)
+                acc = q6k_dot16(rowp + (uint64_t)(c / 16) * GdEnc<ENC>::BYTES, c % 16, x + 16 * c, acc);
 #pragma unroll
         for (int off = 32; off > 0; off >>= 1) acc += __shfl_xor(acc, off, 64);
         float *sums = (float *)lds;
@@ -1144,7 +1173,7 @@ static hipError_t launch_dma(hipStream_t s, const uint8_t *w, uint64_t stride, u
         if (rows < 2) return hipErrorInvalidValue;
         rows -= 1;
     }
-    const uint32_t cus = 256 * wgs_per_cu - (tail ? 1 : 0);
+    uint32_t cus = 256 * wgs_per_cu - (tail ? 1 : 0);
     const uint32_t set_waves = (nblocks + SLOTS - 1) / SLOTS;
     const uint32_t step_rows = 64 / (4 * SLOTS);
     if (set_waves > (uint32_t)gd_threads<ENC>() / 64) return hipErrorInvalidValue;
@@ -1162,6 +1191,13 @@ static hipError_t launch_dma(hipStream_t s, const uint8_t *w, uint64_t stride, u
     // Rows per workgroup need not be whole set steps (each set guards its
     // last step), so the grid is the CU count and each CU streams the same
     // share of the bytes.
+    // The last row's workgroup gets a CU of its own only where no other fits
+    // beside one on it (1024 x 5120: 256 ranges of 4 rows, not 205 of 5).
+    const uint32_t rows_256 = (rows + 256 * wgs_per_cu - 1) / (256 * wgs_per_cu);
+    if (tail && (size_t)set_waves * std::min(sets, std::max(1u, sets_wanted)) * D * GdEnc<ENC>::INSTRS * 1024 +
+                        (size_t)nblocks * 8 * SLICE_WORDS * 4 + (size_t)rows_256 * set_waves * 4 <
+                    72 * 1024)
+        cus += 1;
     const uint32_t rows_per_wg = std::max(1u, (rows + cus - 1) / cus);
     // Fewer wave sets when the rings, x slices and partials exceed the LDS.
     auto lds_for = [&](uint32_t st) {

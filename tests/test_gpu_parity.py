@@ -452,6 +452,31 @@ def test_silu_pair_large_runs_as_two_gemvs(backend, rows):
     assert np.all(np.abs(got - want) <= bound), np.max(np.abs(got - want) - bound)
 
 
+@pytest.mark.parametrize("rows,columns", [(2, 256), (17, 1280), (256, 5120), (257, 5120), (1024, 5120), (1025, 17408),
+                                          (20000, 2304)])
+def test_q6k_last_row_and_row_ranges(backend, rows, columns):
+    """Q6_K rows that end mid-chunk: the last row has a workgroup of its own
+    (16-value groups against F32 x), beside 255 or 256 row ranges; every row,
+    the last ones above all, within the F32 bound, also with an infinity."""
+    import torch
+    w = quantized(14, rows, columns, 61)
+    m = nq.Matrix(14, rows, columns, to_gpu(w))
+    x = gaussian(62, columns)
+    y = torch.full((rows + 1,), np.nan, device="cuda")
+    backend.matvec(m, to_gpu(x), y)
+    backend.sync()
+    got = y.cpu().numpy()
+    assert np.isnan(got[rows])
+    check_close(got[None, :rows], orc.matvec(14, rows, columns, w, x)[None, :], mass(14, w, rows, columns, x[None, :]),
+                F32_K, f"q6k-tail {rows}x{columns}")
+    x[columns // 2 + 3] = np.inf
+    backend.matvec(m, to_gpu(x), y)
+    backend.sync()
+    want = orc.matvec(14, rows, columns, w, x)
+    assert np.array_equal(np.isnan(y[:rows].cpu().numpy()), np.isnan(want))
+    assert np.array_equal(np.isposinf(y[:rows].cpu().numpy()), np.isposinf(want))
+
+
 @pytest.mark.parametrize("encoding,columns,rows", [
     (8, 512, 4096), (8, 17408, 4112), (12, 256, 4112), (12, 17408, 4096), (13, 5120, 4368), (14, 2048, 4352),
     (14, 5120, 4096), (23, 512, 8208), (23, 4096, 4096),
