@@ -635,8 +635,12 @@ static int segments_impl(nuq_context *ctx, const nuq_segment *segments, uint32_t
     // faster as decode GEMVs (gate into the output,
     // up into a workspace) and the elementwise epilogue than as one merged
     // row-per-wave pass.
+    // (also small ones with an encoding that the merged kernel decodes value
+    // by value: Q5_K, IQ4_XS)
+    bool slow = false;
+    for (uint32_t i = 0; i < count; ++i) slow = slow || !specialised(segments[i].matrix.encoding);
     const bool pair_big = mode == NUQ_SEGMENT_SILU_MUL_PAIR && !ctx->generic_only &&
-                          segments[0].matrix.rows >= PAIR_SPLIT_ROWS;
+                          (segments[0].matrix.rows >= PAIR_SPLIT_ROWS || slow);
     const bool pair_split = pair_big && (fixed || ensure_workspace(ctx, segments[0].matrix.rows));
     float *up_buffer = fixed ? fixed : ctx->split.work;
     // Segments of one encoding and row stride (q/k/v, gate/up) run as one
@@ -669,6 +673,15 @@ static int segments_impl(nuq_context *ctx, const nuq_segment *segments, uint32_t
         if (e) return e;
         return hip_check(ctx, nuq::launch_silu_mul(ctx->stream, segments[0].output, up, (uint32_t)g.rows),
                          "silu pair epilogue");
+    }
+    // Plain segments with such an encoding that did not share a launch: each
+    // matrix's own GEMV.
+    if (mode == NUQ_SEGMENT_PLAIN && slow && !ctx->generic_only) {
+        for (uint32_t i = 0; i < count; ++i) {
+            const int e = run_gemv(ctx, &segments[i].matrix, strides[i], x, segments[i].output);
+            if (e) return e;
+        }
+        return NUQ_OK;
     }
     if (mode != NUQ_SEGMENT_PLAIN) args.wave_start[1] = (uint32_t)((segments[0].matrix.rows + rpw - 1) / rpw);
     return hip_check(ctx, nuq::launch_segments(ctx->stream, args, x), "segments launch");

@@ -452,27 +452,29 @@ def test_silu_pair_large_runs_as_two_gemvs(backend, rows):
     assert np.all(np.abs(got - want) <= bound), np.max(np.abs(got - want) - bound)
 
 
-@pytest.mark.parametrize("rows,columns", [(2, 256), (17, 1280), (256, 5120), (257, 5120), (1024, 5120), (1025, 17408),
-                                          (20000, 2304)])
-def test_q6k_last_row_and_row_ranges(backend, rows, columns):
-    """Q6_K rows that end mid-chunk: the last row has a workgroup of its own
-    (16-value groups against F32 x), beside 255 or 256 row ranges; every row,
-    the last ones above all, within the F32 bound, also with an infinity."""
+@pytest.mark.parametrize("encoding,rows,columns", [
+    (14, 2, 256), (14, 17, 1280), (14, 256, 5120), (14, 257, 5120), (14, 1024, 5120), (14, 1025, 17408),
+    (14, 20000, 2304), (23, 2, 256), (23, 17, 1280), (23, 1024, 4864), (23, 257, 17152), (23, 20000, 2304), (23, 1, 768),
+])
+def test_last_row_and_row_ranges(backend, encoding, rows, columns):
+    """Q6_K and IQ4_XS rows that end mid-chunk: the last row has a workgroup
+    of its own (16-value groups against F32 x), beside 255 or 256 row ranges;
+    every row within the F32 bound, also with an infinity."""
     import torch
-    w = quantized(14, rows, columns, 61)
-    m = nq.Matrix(14, rows, columns, to_gpu(w))
+    w = quantized(encoding, rows, columns, 61)
+    m = nq.Matrix(encoding, rows, columns, to_gpu(w))
     x = gaussian(62, columns)
     y = torch.full((rows + 1,), np.nan, device="cuda")
     backend.matvec(m, to_gpu(x), y)
     backend.sync()
     got = y.cpu().numpy()
     assert np.isnan(got[rows])
-    check_close(got[None, :rows], orc.matvec(14, rows, columns, w, x)[None, :], mass(14, w, rows, columns, x[None, :]),
-                F32_K, f"q6k-tail {rows}x{columns}")
+    check_close(got[None, :rows], orc.matvec(encoding, rows, columns, w, x)[None, :],
+                mass(encoding, w, rows, columns, x[None, :]), F32_K, f"last-row {encoding} {rows}x{columns}")
     x[columns // 2 + 3] = np.inf
     backend.matvec(m, to_gpu(x), y)
     backend.sync()
-    want = orc.matvec(14, rows, columns, w, x)
+    want = orc.matvec(encoding, rows, columns, w, x)
     assert np.array_equal(np.isnan(y[:rows].cpu().numpy()), np.isnan(want))
     assert np.array_equal(np.isposinf(y[:rows].cpu().numpy()), np.isposinf(want))
 
@@ -480,7 +482,7 @@ def test_q6k_last_row_and_row_ranges(backend, rows, columns):
 @pytest.mark.parametrize("encoding,columns,rows", [
     (8, 512, 4096), (8, 17408, 4112), (12, 256, 4112), (12, 17408, 4096), (13, 5120, 4368), (14, 2048, 4352),
     (14, 5120, 4096), (23, 512, 8208), (23, 4096, 4096),
-    (8, 4096, 2064), (12, 5120, 16), (13, 2048, 1024), (14, 2048, 272), (23, 512, 48),
+    (8, 4096, 2064), (12, 5120, 16), (13, 2048, 1024), (14, 2048, 272), (23, 512, 48), (23, 768, 32), (23, 3328, 4112),
 ])
 def test_silu_pair_equals_its_gemvs(backend, encoding, columns, rows):
     """The one-launch pair adds each row's sums as that matrix's own matvec
