@@ -91,9 +91,9 @@ void nuq_destroy(nuq_context *ctx);
  * unless either stream is capturing a graph. The previous stream must still
  * be alive when this is called (an event is recorded on it). */
 int nuq_set_stream(nuq_context *ctx, void *stream);
-/* The context's device workspace (verify K-range partials, prefill split
- * partials, the SiLU pair's second GEMV) is allocated on the first call that
- * wants it and grown as needed; nuq_create allocates none. A call that would
+/* The context's device workspace (verify K-range partials, split partial
+ * tiles, the f16 copy of F32 activations, a mixed SiLU pair's second GEMV) is
+ * allocated on the first call that wants it and grown as needed; nuq_create allocates none. A call that would
  * grow it while a graph capture is active takes its no-workspace route
  * instead (same products). A workspace that a captured call used is never
  * freed on growth: it stays allocated until nuq_destroy, so graphs captured

@@ -2355,7 +2355,7 @@ static float prefill_cost(uint32_t rows, uint32_t columns, uint32_t tokens, uint
 }
 
 // At most this much f16 copy of F32 activations at a time (bytes).
-constexpr uint64_t X16_BYTES = 1ull << 30;
+constexpr uint64_t X16_BYTES = 256ull << 20;
 
 // The route of a product on the tiles, with at most max_floats of workspace.
 //  - Q4_K / Q5_K up to VF_PASS_MAX tokens keep the streamed verify tile, whose

@@ -123,3 +123,23 @@ def test_captured_f32_product_replays():
             assert torch.isfinite(y).all()
         b.close()
         b2.close()
+
+
+@pytest.mark.parametrize("encoding,tokens", [(14, 1025), (8, 2051)])
+def test_f32_activations_beyond_one_copy(backend, encoding, tokens):
+    """256 MiB of f16 rows at a time: 1024 rows of 131072 columns, then a
+    short last part."""
+    import torch
+    rows, columns = 72, 131072
+    print(f"[panel] enc {encoding} {rows}x{columns} tokens {tokens} in parts", flush=True)
+    w = nq.quantize(encoding, gaussian(12, (rows, columns), 0.02))
+    m = nq.Matrix(encoding, rows, columns, to_gpu(w))
+    x = torch.randn((tokens, columns), device="cuda", generator=torch.Generator("cuda").manual_seed(8))
+    y = torch.full((tokens, rows), float("nan"), device="cuda")
+    backend.matmul(m, x, columns, y, rows, tokens)
+    backend.sync()
+    check = [0, 1023, 1024, tokens - 1]
+    xr = x[check].half().float().cpu().numpy()
+    assert torch.isfinite(y).all()
+    check_close(y[check].cpu().numpy(), orc.matmul(encoding, rows, columns, w, xr), mass(encoding, w, rows, columns, xr),
+                F16_K, f"panel {encoding} in parts")
