@@ -75,6 +75,23 @@ def test_every_shape_matches_oracle(backend, encoding, shape):
         check_close(got[check, :rows], want, m, F16_K, f"panel {encoding} shape {shape} splits {splits} tail {tail}")
 
 
+@pytest.mark.parametrize("splits", [2, 4, 5, 6, 9, 11])
+def test_partial_sums_of_any_split_count(backend, splits):
+    """The reduction reads four splits at a time: counts around its turns."""
+    import torch
+    rows, tokens, columns = 136, 33, 256 * 11
+    w = nq.quantize(14, gaussian(41, (rows, columns), 0.02))
+    x = gaussian(42, (tokens, columns)).astype(np.float16)
+    wg, xg = to_gpu(w), to_gpu(x)
+    work, y = torch.empty(4 * splits * 32 * 128, device="cuda"), torch.full((tokens, rows), np.nan, device="cuda")
+    args = Args(wg.data_ptr(), w.shape[1], rows, columns, xg.data_ptr(), columns, y.data_ptr(), rows, tokens)
+    assert launch(14, args, Plan(0, 0, 4, splits, 0, 0.0), work.data_ptr()) == 0
+    torch.cuda.synchronize()
+    xr = x.astype(np.float32)
+    check_close(y.cpu().numpy(), orc.matmul(14, rows, columns, w, xr), mass(14, w, rows, columns, xr), F16_K,
+                f"panel {splits} splits")
+
+
 @pytest.mark.parametrize("encoding,rows,columns,tokens", [(12, 1032, 512, 77), (14, 520, 2304, 300), (8, 4104, 2048, 260),
                                                           (8, 264, 320, 40), (23, 8192, 4096, 8)])
 def test_f32_activations_equal_their_f16_rounding(backend, encoding, rows, columns, tokens):
