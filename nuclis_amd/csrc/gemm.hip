@@ -2418,8 +2418,13 @@ void plan_tile(uint32_t encoding, uint32_t rows, uint32_t columns, uint32_t toke
     const uint64_t row_stride = x_f16 ? in_stride : columns;
     const uint64_t split_max = (uint64_t)split_scratch_tiles() * PF_BM * PF_BN;
     const bool room = chunk != 0 && copy <= max_floats;
+    // (a shorter last chunk is planned here too, within the others' partials, so
+    // that none can be refused once another has run)
+    const uint32_t short_chunk = room ? tokens % chunk : 0;
     if (room && panel_plan(encoding, rows, columns, chunk, stride, row_stride, std::min(max_floats - copy, split_max),
-                           &t->panel)) {
+                           &t->panel) &&
+        (short_chunk == 0 ||
+         panel_plan(encoding, rows, columns, short_chunk, stride, row_stride, t->panel.work_floats, &t->last))) {
         const bool both = !small && t->route == TilePlan::PREFILL && encoding == 8;
         if (!both ||
             t->panel.cost < 0.92f * prefill_cost(rows, columns, chunk, std::min(max_floats - copy, split_max))) {
@@ -2519,10 +2524,7 @@ hipError_t launch_tile(hipStream_t s, uint32_t encoding, const uint8_t *w, uint6
             const SplitScratch partials{scratch.work, (uint32_t)(split_floats / (PF_BM * PF_BN))};
             e = launch_prefill_any(s, encoding, w, stride, rows, columns, xc, 1, xs, yc, out_stride, n, partials);
         } else {
-            PanelPlan p = plan.panel;
-            if (n != plan.chunk &&
-                !panel_plan(encoding, rows, columns, n, stride, xs, split_floats, &p))  // a shorter last chunk
-                return hipErrorInvalidValue;
+            const PanelPlan &p = n == plan.chunk ? plan.panel : plan.last;
             e = launch_panel(s, encoding, {w, stride, rows, columns, xc, xs, yc, out_stride, n}, p, scratch.work);
         }
         if (e != hipSuccess) return e;

@@ -79,12 +79,13 @@ hipError_t launch_penalize(hipStream_t s, float *logits, uint32_t count, const u
                            float presence);
 hipError_t launch_topk(hipStream_t s, const float *logits, uint32_t count, uint32_t k, float temperature,
                        uint64_t *scratch, float *values, uint32_t *indices, float *sums, uint32_t *flags);
-// How a product runs on the tiles (plan_tile): the route, its panel plan, the
-// tokens served per chunk, the floats of the f16 copy of F32 activations and
-// the workspace it uses in all (split partials, then the copy).
+// How a product runs on the tiles (plan_tile): the route, its panel plan (and
+// that of a shorter last chunk), the tokens served per chunk, the floats of the
+// f16 copy of F32 activations and the workspace it uses in all (split
+// partials, then the copy).
 struct TilePlan {
     enum Route { VERIFY, PANEL, PREFILL, TILE } route;
-    PanelPlan panel;
+    PanelPlan panel, last;
     uint32_t chunk;
     uint64_t copy, floats;
 };

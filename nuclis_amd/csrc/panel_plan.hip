@@ -111,13 +111,16 @@ bool panel_plan(uint32_t encoding, uint32_t rows, uint32_t columns, uint32_t tok
     if (256 * stride > 0xffffffffull || 256 * in_stride * 2 + 2ull * columns > 0xffffffffull) return false;
     const uint32_t nb = columns / 256;
     const uint32_t groups = (tokens + 31) / 32;
+    // shapes of more token groups than the tokens fill only add padding, and
+    // small ones decode the weights once more per token tile; rows of one
+    // block have no second K set for the three-group shape, so 65 to 96 tokens
+    // pad to four groups there
+    const uint32_t widest = nb == 1 && groups == 3 ? 4 : groups;
     bool found = false;
     for (int i = 0; i < PANEL_SHAPE_COUNT; ++i) {
         const PanelShape &s = PANEL_SHAPES[i];
         const PanelCost &k = PANEL_COST[e][i];
-        // shapes of more token groups than the tokens fill only add padding,
-        // and small ones decode the weights once more per token tile
-        if ((s.tg > groups && s.tg > 1) || (s.tg < 4 && groups > 2u * s.tg) || nb < s.wk) continue;
+        if (s.tg > widest || (s.tg < 4 && groups > 2u * s.tg) || nb < s.wk) continue;
         const uint32_t bm = 32 * s.tg, bn = 32 * s.rg * s.wr, cap = 256 * k.occ;
         const uint64_t tiles64 = (uint64_t)((tokens + bm - 1) / bm) * ((rows + bn - 1) / bn);
         if (tiles64 > 0x7fffffffu / 32) continue;
@@ -151,6 +154,20 @@ bool panel_plan(uint32_t encoding, uint32_t rows, uint32_t columns, uint32_t tok
             for (uint32_t sp = 2; sp <= 4 && sp * s.wk <= nb; ++sp) consider(tiles % cap, sp);
     }
     return found;
+}
+
+// The plan as plain numbers (shape, full, tail, splits, partial floats, then the
+// shape's tokens and rows of a tile and K sets), for checks on the host; 0 when
+// the tile does not take the product.
+extern "C" int nuq_panel_plan(uint32_t encoding, uint32_t rows, uint32_t columns, uint32_t tokens, uint64_t stride,
+                              uint64_t in_stride, uint64_t max_floats, uint64_t out[8]) {
+    PanelPlan p;
+    if (!panel_plan(encoding, rows, columns, tokens, stride, in_stride, max_floats, &p)) return 0;
+    const PanelShape &s = PANEL_SHAPES[p.shape];
+    const uint64_t v[8] = {(uint64_t)p.shape, p.full, p.tail, p.splits, p.work_floats,
+                           32ull * s.tg, 32ull * s.rg * s.wr, s.wk};
+    std::copy(v, v + 8, out);
+    return 1;
 }
 
 // Adds a split tile's partial sums in split order (results do not depend on

@@ -160,3 +160,42 @@ def test_f32_activations_beyond_one_copy(backend, encoding, tokens):
     assert torch.isfinite(y).all()
     check_close(y[check].cpu().numpy(), orc.matmul(encoding, rows, columns, w, xr), mass(encoding, w, rows, columns, xr),
                 F16_K, f"panel {encoding} in parts")
+
+
+@pytest.mark.parametrize("encoding", [8, 12, 13, 14, 23])
+@pytest.mark.parametrize("tokens", [65, 77, 96])
+def test_one_block_rows(backend, encoding, tokens):
+    """Rows of one 256-column block at 65 to 96 tokens: three token groups and
+    no second K set."""
+    import torch
+    rows, columns = 136, 256
+    w = nq.quantize(encoding, gaussian(51, (rows, columns), 0.02))
+    m = nq.Matrix(encoding, rows, columns, to_gpu(w))
+    x = to_gpu(gaussian(52, (tokens, columns)))
+    xr = x.half().float().cpu().numpy()
+    want, ms = orc.matmul(encoding, rows, columns, w, xr), mass(encoding, w, rows, columns, xr)
+    for xg in (x, x.half()):
+        y = torch.full((tokens, rows), float("nan"), device="cuda")
+        backend.matmul(m, xg, columns, y, rows, tokens)
+        backend.sync()
+        check_close(y.cpu().numpy(), want, ms, F16_K, f"panel-one-block {encoding} tokens {tokens}")
+
+
+@pytest.mark.parametrize("encoding", [8, 14])
+def test_one_block_rows_in_parts(backend, encoding):
+    """524288 tokens of 256 columns fill one f16 copy; 77 more are a last part
+    of their own."""
+    import torch
+    rows, columns, tokens = 8, 256, 524288 + 77
+    print(f"[panel] enc {encoding} {rows}x{columns} tokens {tokens} in parts", flush=True)
+    w = nq.quantize(encoding, gaussian(53, (rows, columns), 0.02))
+    m = nq.Matrix(encoding, rows, columns, to_gpu(w))
+    x = torch.randn((tokens, columns), device="cuda", generator=torch.Generator("cuda").manual_seed(9))
+    y = torch.full((tokens, rows), float("nan"), device="cuda")
+    backend.matmul(m, x, columns, y, rows, tokens)
+    backend.sync()
+    assert torch.isfinite(y).all()
+    check = [0, 524287, 524288, tokens - 1]
+    xr = x[check].half().float().cpu().numpy()
+    check_close(y[check].cpu().numpy(), orc.matmul(encoding, rows, columns, w, xr), mass(encoding, w, rows, columns, xr),
+                F16_K, f"panel-one-block {encoding} in parts")
