@@ -17,11 +17,10 @@
 //  - activations XOR-swizzled in 16-byte chunks over row pairs: no bank
 //    conflicts on fragment reads (two-way before: 44 M conflict cycles of
 //    96 M, 710 -> 702 us).
-//  - scales unpacked once per unit, codes into the mantissa of 1024.0 by one
-//    v_and_or_b32 per pair and the bias folded into the F32 addend of
-//    v_fma_mix: 1.6 VALU operations a weight; and the hand-over to the next
-//    slab (wait, barrier, copies, first fragment reads) under the last
-//    sub-step's products: 702 -> 683 us.
+//  - scales unpacked once per unit, codes into f16 by one masking operation per
+//    pair and one v_fma_mix a weight: 1.6 VALU operations a weight; and the
+//    hand-over to the next slab (wait, barrier, copies, first fragment reads)
+//    under the last sub-step's products: 702 -> 683 us.
 // At 4096 tokens the card is power-limited (1.5-1.6 GHz at 60 % MFMA
 // occupancy against 1.8 GHz at 53 % in the LDS-staged tile), so fewer VALU and
 // LDS operations per product count more than fewer stalls. 4096 tokens: 748 ->
@@ -52,33 +51,67 @@ __device__ __forceinline__ uint32_t and_or(uint32_t t, uint32_t o) {
     return r;
 }
 
-// Two f16 values 1024 + code from the halves of t (codes below 1024): the
-// masked bits go into the mantissa of 1024.0, whose ulp is 1. The second
-// form takes more code bits from u.
+// The weights are the CPU decoders' values rounded to f16, also where a block's
+// scale is infinite: +-Inf by the code's sign, NaN for a zero code. Unsigned
+// codes (Q4_K, Q5_K) are read as f16 subnormals, code 2^-24, by one and (or one
+// byte permute) per pair, with 2^24 in the scale.
+template <uint32_t M>
+__device__ __forceinline__ half2v subnormal(uint32_t t) {
+    return __builtin_bit_cast(half2v, opaque_and<M>(t));
+}
+// from bytes I and I + 2 of t
+template <uint32_t I>
+__device__ __forceinline__ half2v subnormal_bytes(uint32_t t) {
+    return __builtin_bit_cast(half2v, __builtin_amdgcn_perm(0u, t, 0x0c020c00u + 0x00010001u * I));
+}
+// Signed codes of Q6_K and IQ4_XS carry a bias: two f16 values 1024 + byte (the
+// byte goes into the mantissa of 1024.0, whose ulp is 1), whose bias the F32
+// addend takes out. The addend is exact (the scale has at most 18 bits, the
+// bias 6), but infinite with the scale: infinite scales are replaced
+// (overflowing) before.
 constexpr uint32_t F16_1024 = 0x64006400u;
 template <uint32_t M>
 __device__ __forceinline__ half2v biased(uint32_t t) {
     return __builtin_bit_cast(half2v, and_or<M>(t, F16_1024));
 }
-// Two f16 values 1024 + byte from bytes I and I + 2 of t.
+// from bytes I and I + 2 of t
 template <uint32_t I>
 __device__ __forceinline__ half2v biased_bytes(uint32_t t) {
     return __builtin_bit_cast(half2v, __builtin_amdgcn_perm(F16_1024 | 0x00640064u, t, 0x04020400u + 0x00010001u * I));
 }
+// A finite value of v's sign in the place of +-Inf, whose products with codes
+// other than zero overflow f16 to +-Inf again.
+__device__ __forceinline__ float overflowing(float v) {
+    return fabsf(v) == INFINITY ? copysignf(0x1p100f, v) : v;
+}
 
-// f16(v * mul + add), one rounding (v_fma_mix). v carries a bias of 1024 (+ 32
-// or 128), add takes it out: exact for Q6_K, Q8_0 and IQ4_XS (mul has at most 18
-// bits, the bias 6), so zero weights stay zero; for Q4_K and Q5_K add is rounded
-// to 2^-15 of mul, under a tenth of the weight's own f16 rounding.
+// f16(v * mul + add), one F32 rounding before it (v_fma_mix): the value of the
+// CPU decoders' product-sum.
 __device__ __forceinline__ _Float16 mix(_Float16 v, float mul, float add) { return (_Float16)fmaf((float)v, mul, add); }
 
-// Four weights of one code word: `even` holds 1024 + codes of bytes 0 and 2,
+// Four weights of one code word: `even` holds the codes of bytes 0 and 2,
 // `odd` of bytes 1 and 3.
 __device__ __forceinline__ void four(half8 &f, int at, half2v even, half2v odd, float mul, float add) {
     f[at] = mix(even[0], mul, add);
     f[at + 1] = mix(odd[0], mul, add);
     f[at + 2] = mix(even[1], mul, add);
     f[at + 3] = mix(odd[1], mul, add);
+}
+// Four weights from the signed bytes of t. `zero` is an f16 zero the compiler
+// cannot see through: with it the product and its rounding are one v_fma_mix
+// (a plain product is rounded by a second instruction). One conversion a code
+// takes the place of the biased form's masks, so Q8_0 needs no bias: 17408 x
+// 5120 at 4096 tokens 735-737 us against 730-737.
+__device__ __forceinline__ void four_signed(half8 &f, int at, uint32_t t, float mul, _Float16 zero) {
+    f[at] = (_Float16)fmaf(sbyte_f<0>(t), mul, (float)zero);
+    f[at + 1] = (_Float16)fmaf(sbyte_f<1>(t), mul, (float)zero);
+    f[at + 2] = (_Float16)fmaf(sbyte_f<2>(t), mul, (float)zero);
+    f[at + 3] = (_Float16)fmaf(sbyte_f<3>(t), mul, (float)zero);
+}
+__device__ __forceinline__ _Float16 opaque_zero() {
+    uint32_t z = 0;
+    asm("" : "+s"(z));
+    return __builtin_bit_cast(half2v, z)[0];
 }
 
 // The eight 6-bit scales and minima of a Q4_K / Q5_K header as bytes (groups
@@ -108,7 +141,7 @@ struct PanelRaw<12> {
     static constexpr uint32_t SLABS = 4, BYTES = 144, NCH = 9, NX = 0, UNITS = 1;
     u32x4 hdr, qs[4];
     uint32_t sc[2], mn[2];
-    float d, d16, ndmin, mul0, add0, mul1, add1;
+    float d24, d20, ndmin, mul0, add0, mul1, add1;
     __device__ static uint32_t src(uint32_t c) { return 16 * c; }
     __device__ static uint32_t chunk_of(uint32_t c, uint32_t part) { return (c & 1) * 4 + part * 2 + (c >> 1); }
     __device__ __forceinline__ void read(const uint8_t *unit, const uint8_t *, uint32_t part) {
@@ -117,16 +150,18 @@ struct PanelRaw<12> {
         for (int p = 0; p < 4; ++p) qs[p] = *(const u32x4 *)(unit + part * 16 + 16 + 32 * p);
     }
     __device__ __forceinline__ void open() {
+        float d;
         open_k(hdr, sc, mn, d, ndmin);
-        d16 = d * 0.0625f;
+        d24 = d * 0x1p24f;
+        d20 = d * 0x1p20f;  // high nibbles stay in place (16 q)
     }
     template <int P>
     __device__ __forceinline__ void setup(uint32_t) {
         constexpr int E = 2 * (P & 1);
-        mul0 = d * ubyte_f<E>(sc[P >> 1]);
-        mul1 = d16 * ubyte_f<E + 1>(sc[P >> 1]);  // d / 16: high nibbles stay in place (16 q)
-        add0 = fmaf(mul0, -1024.f, ndmin * ubyte_f<E>(mn[P >> 1]));
-        add1 = fmaf(mul1, -1024.f, ndmin * ubyte_f<E + 1>(mn[P >> 1]));
+        mul0 = d24 * ubyte_f<E>(sc[P >> 1]);
+        mul1 = d20 * ubyte_f<E + 1>(sc[P >> 1]);
+        add0 = ndmin * ubyte_f<E>(mn[P >> 1]);
+        add1 = ndmin * ubyte_f<E + 1>(mn[P >> 1]);
     }
     template <int P, int C>
     __device__ __forceinline__ half8 chunk() const {
@@ -135,9 +170,9 @@ struct PanelRaw<12> {
         for (int k = 0; k < 2; ++k) {
             const uint32_t t = qs[P][2 * (C >> 1) + k];
             if constexpr ((C & 1) == 0)
-                four(f, 4 * k, biased<0x000f000fu>(t), biased<0x000f000fu>(t >> 8), mul0, add0);
+                four(f, 4 * k, subnormal<0x000f000fu>(t), subnormal<0x000f000fu>(t >> 8), mul0, add0);
             else
-                four(f, 4 * k, biased<0x00f000f0u>(t), biased<0x00f000f0u>(t >> 8), mul1, add1);
+                four(f, 4 * k, subnormal<0x00f000f0u>(t), subnormal<0x00f000f0u>(t >> 8), mul1, add1);
         }
         return f;
     }
@@ -148,7 +183,7 @@ struct PanelRaw<13> {
     static constexpr uint32_t SLABS = 4, BYTES = 176, NCH = 11, NX = 0, UNITS = 1;
     u32x4 hdr, qh, qs[4];
     uint32_t sc[2], mn[2];
-    float d, ndmin, mul0, add0, mul1, add1;
+    float d24, ndmin, mul0, add0, mul1, add1;
     __device__ static uint32_t src(uint32_t c) { return 16 * c; }
     __device__ static uint32_t chunk_of(uint32_t c, uint32_t part) { return (c & 1) * 4 + part * 2 + (c >> 1); }
     __device__ __forceinline__ void read(const uint8_t *unit, const uint8_t *, uint32_t part) {
@@ -158,15 +193,17 @@ struct PanelRaw<13> {
         for (int p = 0; p < 4; ++p) qs[p] = *(const u32x4 *)(unit + part * 16 + 48 + 32 * p);
     }
     __device__ __forceinline__ void open() {
+        float d;
         open_k(hdr, sc, mn, d, ndmin);
+        d24 = d * 0x1p24f;
     }
     template <int P>
     __device__ __forceinline__ void setup(uint32_t) {
         constexpr int E = 2 * (P & 1);
-        mul0 = d * ubyte_f<E>(sc[P >> 1]);
-        mul1 = d * ubyte_f<E + 1>(sc[P >> 1]);
-        add0 = fmaf(mul0, -1024.f, ndmin * ubyte_f<E>(mn[P >> 1]));
-        add1 = fmaf(mul1, -1024.f, ndmin * ubyte_f<E + 1>(mn[P >> 1]));
+        mul0 = d24 * ubyte_f<E>(sc[P >> 1]);
+        mul1 = d24 * ubyte_f<E + 1>(sc[P >> 1]);
+        add0 = ndmin * ubyte_f<E>(mn[P >> 1]);
+        add1 = ndmin * ubyte_f<E + 1>(mn[P >> 1]);
     }
     template <int P, int C>
     __device__ __forceinline__ half8 chunk() const {
@@ -178,12 +215,12 @@ struct PanelRaw<13> {
                 // bit 2P of every high byte to bit 4
                 const uint32_t b = 2 * P <= 4 ? h << (4 - 2 * P) : h >> (2 * P - 4);
                 const uint32_t u = and_or<0x10101010u>(b, opaque_and<0x0f0f0f0fu>(t));
-                four(f, 4 * k, biased_bytes<0>(u), biased_bytes<1>(u), mul0, add0);
+                four(f, 4 * k, subnormal_bytes<0>(u), subnormal_bytes<1>(u), mul0, add0);
             } else {
                 // bit 2P + 1 to bit 4
                 const uint32_t b = 2 * P + 1 <= 4 ? h << (3 - 2 * P) : h >> (2 * P - 3);
                 const uint32_t u = and_or<0x10101010u>(b, opaque_and<0x0f0f0f0fu>(t >> 4));
-                four(f, 4 * k, biased_bytes<0>(u), biased_bytes<1>(u), mul1, add1);
+                four(f, 4 * k, subnormal_bytes<0>(u), subnormal_bytes<1>(u), mul1, add1);
             }
         }
         return f;
@@ -234,6 +271,21 @@ struct PanelRaw<14> {
         }
         return f;
     }
+    // An infinite d, from the row's image: NaN if any weight of the block is (a
+    // zero code or scale; its other weights only meet outputs that are NaN with
+    // it), else a value that overflows. A rolled loop: unrolled over the
+    // registers it would cost the main loop half its waves.
+    __device__ __forceinline__ void settle(const uint8_t *unit) {
+        if (fabsf(d) != INFINITY) return;
+        bool zero = false;
+#pragma unroll 1
+        for (uint32_t k = 0; k < 128; ++k) {
+            const uint32_t l = unit[k], h = unit[128 + (k >> 6) * 32 + (k & 31)] >> (2 * ((k >> 5) & 1));
+            zero = zero || ((l & 15u) | (h & 3u) << 4) == 32u || (l >> 4 | ((h >> 4) & 3u) << 4) == 32u ||
+                   unit[192 + (k & 15)] == 0;
+        }
+        d = zero ? NAN : overflowing(d);
+    }
 };
 
 // IQ4_XS: chunk 0 is the header (and the first codes again), chunk 1 + g group g
@@ -255,7 +307,7 @@ struct PanelRaw<23> {
     __device__ __forceinline__ void setup(uint32_t part) {
         const uint32_t low = (hdr.y >> (8 * P + 4 * part)) & 15u;
         const int sc = (int)(low | (((hdr.x >> (16 + 4 * P + 2 * part)) & 3u) << 4)) - 32;
-        mul = half_bits(hdr.x & 0xffffu) * (float)sc;
+        mul = overflowing(half_bits(hdr.x & 0xffffu) * (float)sc);  // no code is zero; Inf x 0 stays NaN
         add = mul * -1152.f;
     }
     template <int P, int C>
@@ -279,7 +331,7 @@ struct PanelRaw<8> {
     static constexpr uint32_t SLABS = 2, BYTES = 136, NCH = 8, NX = 4, UNITS = 2;
     u32x4 qa[2], qb[2];
     uint32_t d16[2];
-    float mul, add;
+    float mul;
     __device__ __forceinline__ void open() {}
     __device__ static uint32_t src(uint32_t c) { return c / 2 * 34 + 2 + c % 2 * 16; }
     __device__ static uint32_t src_dword(uint32_t q) { return 34 * q; }
@@ -296,16 +348,13 @@ struct PanelRaw<8> {
     template <int P>
     __device__ __forceinline__ void setup(uint32_t) {
         mul = half_bits(d16[P] & 0xffffu);
-        add = mul * -1152.f;
     }
     template <int P, int C>
     __device__ __forceinline__ half8 chunk() const {
         half8 f;
 #pragma unroll
-        for (int k = 0; k < 2; ++k) {
-            const uint32_t v = ((C >> 1) == 0 ? qa[P][2 * (C & 1) + k] : qb[P][2 * (C & 1) + k]) ^ 0x80808080u;
-            four(f, 4 * k, biased<0x00ff00ffu>(v), biased<0x00ff00ffu>(v >> 8), mul, add);
-        }
+        for (int k = 0; k < 2; ++k)
+            four_signed(f, 4 * k, (C >> 1) == 0 ? qa[P][2 * (C & 1) + k] : qb[P][2 * (C & 1) + k], mul, opaque_zero());
         return f;
     }
 };
@@ -521,6 +570,21 @@ __global__ void __launch_bounds__(64 * WR * WK, (panel_waves<ENC, TG, RG, WR, WK
         if constexpr (FENCE) __builtin_amdgcn_sched_barrier(0);                                                \
     }
     for (uint32_t ks = ks0; ks < ks1; ks += 4) {
+        // an infinite Q6_K scale in the unit just opened: a wave-uniform
+        // branch where the loop turns, outside the schedule of the steps
+        if constexpr (ENC == 14) {
+            bool inf = false;
+#pragma unroll
+            for (int g = 0; g < RG; ++g) inf = inf || fabsf(raw[g].d) == INFINITY;
+            if (__builtin_amdgcn_ballot_w64(inf) != 0) {
+#pragma unroll
+                for (int g = 0; g < RG; ++g) {
+                    raw[g].settle(image + g * 32 * ROWB);
+                    raw[g].template setup<0>(part);
+                    fb[0][g] = raw[g].template chunk<0, 0>();
+                }
+            }
+        }
         PN_STEP(0)
         PN_STEP(1)
         PN_STEP(2)

@@ -75,6 +75,116 @@ def test_every_shape_matches_oracle(backend, encoding, shape):
         check_close(got[check, :rows], want, m, F16_K, f"panel {encoding} shape {shape} splits {splits} tail {tail}")
 
 
+def run_shape(encoding, shape, w, x, splits=1):
+    """The product on one forced shape: [tokens][rows]."""
+    import torch
+    tg, rg, wr, wk, _ = SHAPES[shape]
+    bm, bn = 32 * tg, 32 * rg * wr
+    rows, tokens, columns = w.shape[0], *x.shape
+    tiles = -(-tokens // bm) * -(-rows // bn)
+    wg, xg, y = to_gpu(w), to_gpu(x), torch.full((tokens, rows), float("nan"), device="cuda")
+    work = torch.empty(tiles * splits * bm * bn, device="cuda")
+    args = Args(wg.data_ptr(), w.shape[1], rows, columns, xg.data_ptr(), columns, y.data_ptr(), rows, tokens)
+    plan = Plan(shape, tiles, 0, 1, 0, 0.0) if splits == 1 else Plan(shape, 0, tiles, splits, 0, 0.0)
+    assert launch(encoding, args, plan, work.data_ptr()) == 0
+    torch.cuda.synchronize()
+    return y.cpu().numpy()
+
+
+@pytest.mark.parametrize("shape", range(len(SHAPES)))
+@pytest.mark.parametrize("encoding", [8, 12, 13, 14, 23])
+def test_weights_are_the_decoded_values_in_f16(backend, encoding, shape):
+    """Every weight is the CPU decoder's F32 value rounded to f16 and nothing
+    else, so against those weights in float64 only the F32 sums are left:
+    activations of a non-zero mean show an offset that a group shares."""
+    wk = SHAPES[shape][3]
+    rows, tokens, columns = 200, 40, 256 * max(2, wk)
+    print(f"[panel-exact] enc {encoding} shape {shape}", flush=True)
+    w = nq.quantize(encoding, gaussian(61 + shape, (rows, columns), 0.02))
+    x = (gaussian(62, (tokens, columns)) + 1).astype(np.float16)
+    dec = orc.decode_matrix(encoding, w, rows, columns).astype(np.float16).astype(np.float64)
+    got = run_shape(encoding, shape, w, x)
+    want, m = x.astype(np.float64) @ dec.T, np.abs(x.astype(np.float64)) @ np.abs(dec).T
+    # at most columns / 16 + 4 F32 roundings of a running sum (16 products of
+    # the matrix core's inner sum, the K sets and halves), each of at most
+    # 2^-24 of the mass; the core's own alignment of 16 products adds as much
+    bound = 2 * (columns / 16 + 4) * 2.0**-24 * m
+    assert (np.abs(got - want) <= bound).all(), float((np.abs(got - want) / m).max())
+
+
+def blocks(encoding, rows, columns, seed):
+    """Random blocks with ordinary scales: [rows][blocks][block bytes]."""
+    values, size = nq.LAYOUT[encoding]
+    return nq.quantize(encoding, gaussian(seed, (rows, columns), 0.02)).reshape(rows, columns // values, size).copy()
+
+
+@pytest.mark.parametrize("shape", range(len(SHAPES)))
+@pytest.mark.parametrize("encoding", [12, 13])
+def test_zero_weights_meet_infinity(backend, encoding, shape):
+    """A weight of exactly zero (d sc q = dmin m) times an infinite activation
+    is NaN, as in the CPU reference; all other rows give an infinity."""
+    rows, tokens, columns = 200, 40, 256 * max(2, SHAPES[shape][3])
+    b = blocks(encoding, rows, columns, 71)
+    b[..., 2:4] = b[..., 0:2] = np.random.default_rng(72).integers(0x1800, 0x2400, b.shape[:2], dtype=np.uint16)[..., None].view(np.uint8)
+    w = b.reshape(rows, -1)
+    dec = orc.decode_matrix(encoding, w, rows, columns)
+    x = np.ones((tokens, columns), np.float16)
+    cols = np.argsort(-(dec == 0).sum(0))[:tokens]  # the columns with most zeros
+    x[np.arange(tokens), cols] = np.inf
+    want_nan = (dec[:, cols] == 0).T
+    assert want_nan.any() and not want_nan.all()
+    got = run_shape(encoding, shape, w, x)
+    assert np.array_equal(np.isnan(got), want_nan)
+    assert np.array_equal(np.isposinf(got), (dec[:, cols] > 0).T) and np.array_equal(np.isneginf(got), (dec[:, cols] < 0).T)
+
+
+@pytest.mark.parametrize("shape", range(len(SHAPES)))
+@pytest.mark.parametrize("encoding", [8, 12, 13, 14, 23])
+def test_infinite_scales_keep_the_weights_signs(backend, encoding, shape):
+    """A block of infinite scale: +-Inf for codes of one sign, NaN for a zero
+    code (rows 1 mod 4) and for a scale of zero (rows 2 mod 4); rows 0 mod 4
+    are finite."""
+    rows, tokens, columns = 200, 40, 256 * max(2, SHAPES[shape][3])
+    values, _ = nq.LAYOUT[encoding]
+    b = blocks(encoding, rows, columns, 81)
+    sick = np.arange(rows) % 4 != 0
+    at = (columns // values) - 1  # in the last block, also a unit's second half for Q8_0
+    d = {8: 0, 12: 0, 13: 0, 14: 208, 23: 0}[encoding]
+    sign = np.where(np.arange(rows) % 8 == 3, 0x7c00, 0xfc00).astype(np.uint16)
+    blk = b[:, at]
+    if encoding == 8:
+        blk[:, 2:] = 5
+        blk[1::4, 9] = 0
+        blk[2::4, 2:] = 0
+    elif encoding in (12, 13):
+        blk[:, 2:4] = 0                       # dmin = 0
+        blk[:, 4:16] = 0x2f
+        blk[:, -128:] |= 0x11                 # no zero code
+        blk[1::4, -128 + 37] = 0
+        if encoding == 13:
+            blk[1::4, 16:48] = 0
+        blk[2::4, 4:16] = 0
+    elif encoding == 14:
+        blk[:, :128], blk[:, 128:192], blk[:, 192:208] = 0x55, 0xaa, 3   # codes 37
+        blk[1::4, 77] = 0x50                  # one code of 32
+        blk[2::4, 199] = 0
+    else:
+        blk[:, 2:4], blk[:, 4:8] = 0xff, 0x11
+        blk[:, 8:] |= 0x88                    # positive values
+        blk[2::4, 2:4], blk[2::4, 4:8] = 0xaa, 0x00  # scales of zero
+    blk[sick, d:d + 2] = sign[sick].view(np.uint8).reshape(-1, 2)
+    w = b.reshape(rows, -1)
+    dec = orc.decode_matrix(encoding, w, rows, columns).astype(np.float64)
+    x = np.abs(gaussian(82, (tokens, columns))).astype(np.float16) + np.float16(0.5)
+    with np.errstate(invalid="ignore"):
+        want = (dec[None] * x.astype(np.float64)[:, None, :]).sum(-1)
+    assert np.isposinf(want).any() and np.isneginf(want).any() and np.isnan(want).any()
+    assert np.isfinite(want[:, ~sick]).all()
+    got = run_shape(encoding, shape, w, x)
+    for cls in (np.isnan, np.isposinf, np.isneginf):
+        assert np.array_equal(cls(got), cls(want)), cls.__name__
+
+
 @pytest.mark.parametrize("splits", [2, 4, 5, 6, 9, 11])
 def test_partial_sums_of_any_split_count(backend, splits):
     """The reduction reads four splits at a time: counts around its turns."""
