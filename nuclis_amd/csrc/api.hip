@@ -192,7 +192,8 @@ int gemv_rows_per_wave(uint32_t encoding, uint64_t rows) {
 
 // The decode GEMV: every encoding on the integer-dot DMA kernel where its
 // shape fits (Q8_0 needs K % 256 == 0), else the register kernel (Q4_K), the
-// row-per-wave kernels (Q6_K, Q8_0) or the generic kernel (Q5_K, IQ4_XS).
+// row-per-wave kernels (the others; IQ4_XS rows of an odd block count, which end
+// mid-chunk: 10027 x 7424 29 us, 199 on the generic kernel).
 int run_gemv(nuq_context *ctx, const nuq_matrix *m, uint64_t stride, const float *x, float *out) {
     if (m->encoding == NUQ_Q6_K || m->encoding == NUQ_Q8_0) {
         hipError_t e = nuq::launch_gemv_dma(ctx->stream, m->encoding, (const uint8_t *)m->bytes, stride,
@@ -204,10 +205,9 @@ int run_gemv(nuq_context *ctx, const nuq_matrix *m, uint64_t stride, const float
                                             (uint32_t)m->rows, (uint32_t)m->columns, x, out);
         if (e != hipErrorInvalidValue) return hip_check(ctx, e, "gemv launch");
         return hip_check(ctx,
-                         nuq::launch_generic(ctx->stream, m->encoding, (const uint8_t *)m->bytes, stride,
-                                             (uint32_t)m->rows, (uint32_t)m->columns, x, 0, m->columns, out, m->rows,
-                                             1),
-                         "generic kernel launch");
+                         nuq::launch_rows_f32(ctx->stream, m->encoding, (const uint8_t *)m->bytes, stride,
+                                              (uint32_t)m->rows, (uint32_t)m->columns, x, out),
+                         "gemv launch");
     }
     if (m->encoding == NUQ_Q4_K) {
         const int config = 0;  // DMA kernel, two ring slots; register kernel when LDS is short
@@ -557,7 +557,7 @@ int nuq_gemm(nuq_context *ctx, uint32_t encoding, const void *w, uint64_t stride
     return nuq_matmul(ctx, &m, x, x_dtype, in_stride, y, out_stride, tokens);
 }
 
-// Rows from which a SiLU pair runs as two decode GEMVs plus the epilogue.
+// Rows from which a SiLU pair runs on the decode GEMV.
 constexpr uint64_t PAIR_SPLIT_ROWS = 4096;
 
 // The body of both segment entry points. `fixed` (the allocation-free form)
@@ -619,28 +619,27 @@ static int segments_impl(nuq_context *ctx, const nuq_segment *segments, uint32_t
     bool same = !ctx->generic_only;
     for (uint32_t i = 1; i < count && same; ++i)
         same = segments[i].matrix.encoding == segments[0].matrix.encoding && strides[i] == strides[0];
-    // A SiLU pair of one encoding is one launch of the decode GEMV with the
-    // epilogue on its own sums, at any row count: 1024 x 5120 / 2048 x 8192
-    // take 7.2 / 7.3-9 us on MI355X, on the merged row kernel below 10 / 14 us
-    // (Q4_K, Q6_K), 12 / 17 (Q8_0) and, without a row kernel of their own,
-    // 197 / 364 (Q5_K) and 120 / 219 (IQ4_XS).
-    if (same && mode == NUQ_SEGMENT_SILU_MUL_PAIR) {
+    // A large SiLU pair of one encoding is one launch of the decode GEMV with
+    // the epilogue on its own sums. Smaller pairs keep the merged kernel's F32
+    // activations: the GEMV's
+    // 23-bit fixed point has 1.5 to 2.5 times the merged kernel's error against
+    // float64 for Q4_K, 3 to 5 times for Q5_K, 1.0 to 1.7 times for Q6_K and 1.6
+    // for IQ4_XS (16..4080 rows of 2048..8192 columns; 1024 x 5120 takes 8.3 us
+    // on it and 8.4 to 13 merged). Q8_0 has 0.8 to 1.0 times the error there and
+    // takes the one launch at any row count (2048 x 8192 17 us merged, 8.4 here).
+    if (same && mode == NUQ_SEGMENT_SILU_MUL_PAIR &&
+        (segments[0].matrix.rows >= PAIR_SPLIT_ROWS || segments[0].matrix.encoding == NUQ_Q8_0)) {
         const nuq_matrix &g = segments[0].matrix;
         const hipError_t he = nuq::launch_gemv_dma_pair(ctx->stream, g.encoding, (const uint8_t *)g.bytes,
                                                         (const uint8_t *)segments[1].matrix.bytes, strides[0],
                                                         (uint32_t)g.rows, (uint32_t)columns, x, segments[0].output);
         if (he != hipErrorInvalidValue) return hip_check(ctx, he, "silu pair launch");
     }
-    // Other large pairs (mixed encodings, Q6_K rows that end mid-chunk) stream
-    // faster as decode GEMVs (gate into the output,
-    // up into a workspace) and the elementwise epilogue than as one merged
-    // row-per-wave pass.
-    // (also small ones with an encoding that the merged kernel decodes value
-    // by value: Q5_K, IQ4_XS)
-    bool slow = false;
-    for (uint32_t i = 0; i < count; ++i) slow = slow || !specialised(segments[i].matrix.encoding);
+    // Other large pairs (mixed encodings, rows that end mid-chunk) stream faster
+    // as decode GEMVs (gate into the output, up into a workspace) and the
+    // elementwise epilogue than as one merged row-per-wave pass.
     const bool pair_big = mode == NUQ_SEGMENT_SILU_MUL_PAIR && !ctx->generic_only &&
-                          (segments[0].matrix.rows >= PAIR_SPLIT_ROWS || slow);
+                          segments[0].matrix.rows >= PAIR_SPLIT_ROWS;
     const bool pair_split = pair_big && (fixed || ensure_workspace(ctx, segments[0].matrix.rows));
     float *up_buffer = fixed ? fixed : ctx->split.work;
     // Segments of one encoding and row stride (q/k/v, gate/up) run as one
@@ -673,15 +672,6 @@ static int segments_impl(nuq_context *ctx, const nuq_segment *segments, uint32_t
         if (e) return e;
         return hip_check(ctx, nuq::launch_silu_mul(ctx->stream, segments[0].output, up, (uint32_t)g.rows),
                          "silu pair epilogue");
-    }
-    // Plain segments with such an encoding that did not share a launch: each
-    // matrix's own GEMV.
-    if (mode == NUQ_SEGMENT_PLAIN && slow && !ctx->generic_only) {
-        for (uint32_t i = 0; i < count; ++i) {
-            const int e = run_gemv(ctx, &segments[i].matrix, strides[i], x, segments[i].output);
-            if (e) return e;
-        }
-        return NUQ_OK;
     }
     if (mode != NUQ_SEGMENT_PLAIN) args.wave_start[1] = (uint32_t)((segments[0].matrix.rows + rpw - 1) / rpw);
     return hip_check(ctx, nuq::launch_segments(ctx->stream, args, x), "segments launch");

@@ -833,27 +833,6 @@ __device__ __forceinline__ float q6k_dot16(const uint8_t *blk, uint32_t s, const
     return acc;
 }
 
-// The same for IQ4_XS: the low (s even) or high nibbles of group s / 2's bytes.
-__device__ __forceinline__ float iq4_dot16(const uint8_t *blk, uint32_t s, const float *__restrict__ x, float acc) {
-    const uint32_t g = s >> 1;
-    const uint2 hdr = *(const uint2 *)blk, qa = *(const uint2 *)(blk + 8 + 16 * g), qb = *(const uint2 *)(blk + 16 + 16 * g);
-    const uint32_t q[4] = {qa.x, qa.y, qb.x, qb.y};
-    float4 xv[4];
-#pragma unroll
-    for (int k = 0; k < 4; ++k) xv[k] = ((const float4 *)x)[k];
-    const uint32_t low = (hdr.y >> (8 * (g / 2) + 4 * (g % 2))) & 15u;
-    const float mul = half_bits(hdr.x & 0xffffu) * (float)((int)(low | (((hdr.x >> (16 + 2 * g)) & 3u) << 4)) - 32);
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        const uint32_t v = iq4_lookup((q[k] >> (4 * (s & 1))) & 0x0f0f0f0fu);
-        acc = fmaf(mul * sbyte_f<0>(v), xv[k].x, acc);
-        acc = fmaf(mul * sbyte_f<1>(v), xv[k].y, acc);
-        acc = fmaf(mul * sbyte_f<2>(v), xv[k].z, acc);
-        acc = fmaf(mul * sbyte_f<3>(v), xv[k].w, acc);
-    }
-    return acc;
-}
-
 // Workgroup size cap of the DMA kernel: 16 waves, except Q6_K, whose lanes
 // hold more bytes per block (the alignment shifts) and so take 12 waves,
 // keeping its registers (up to 170) clear of spills.
@@ -902,9 +881,9 @@ __global__ void __launch_bounds__(gd_threads<ENC>()) gemv_dma_kernel(const uint8
         // than the others of a small matrix: 1024 x 5120 9.4 us in all).
         const uint8_t *rowp = w + (uint64_t)rows * stride;
         float acc = 0.f;
-        if constexpr (ENC == 14 || ENC == 23)
+        if constexpr (ENC == 14)
             for (uint32_t c = threadIdx.x; c < nblocks * 16; c += blockDim.x)
-                acc = (ENC == 14 ? q6k_dot16 : iq4_dot16)(rowp + (uint64_t)(c / 16) * GdEnc<ENC>::BYTES, c % 16, x + 16 * c, acc);
+                acc = q6k_dot16(rowp + (uint64_t)(c / 16) * GdEnc<ENC>::BYTES, c % 16, x + 16 * c, acc);
 #pragma unroll
         for (int off = 32; off > 0; off >>= 1) acc += __shfl_xor(acc, off, 64);
         float *sums = (float *)lds;
@@ -1405,8 +1384,9 @@ hipError_t launch_gemv_q4k_int(hipStream_t s, const uint8_t *w, uint64_t stride,
 // Q5_K / Q6_K / IQ4_XS decode GEMV on the DMA kernel (two ring slots; Q6_K
 // always with 8-block lane groups, so a row's segment is whole chunks). Returns
 // hipErrorInvalidValue when the shape does not fit (more than 128 blocks per
-// row, x and the rings beyond LDS, or a one-row matrix whose row ends
-// mid-chunk): the caller then uses the generic kernel.
+// row, x and the rings beyond LDS, a one-row matrix whose row ends mid-chunk, or
+// IQ4_XS rows of an odd block count, whose 136-byte blocks would end mid-chunk):
+// the caller then uses an F32 kernel.
 hipError_t launch_gemv_dma(hipStream_t s, uint32_t encoding, const uint8_t *w, uint64_t stride, uint32_t rows,
                            uint32_t columns, const float *x, float *y) {
     const uint32_t nblocks = columns / 256;
@@ -1423,12 +1403,9 @@ hipError_t launch_gemv_dma(hipStream_t s, uint32_t encoding, const uint8_t *w, u
     if (encoding == 8 && columns % 256 == 0)  // nblocks counts 256-value units of eight Q8_0 blocks
         return four ? launch_dma<8, 4, 2>(s, w, stride, rows, nblocks, x, y, 0, 1)
                     : launch_dma<8, 8, 2>(s, w, stride, rows, nblocks, x, y, 0, 1);
-    if (encoding == 23)
-        // a row of an odd block count ends mid-chunk too (its last copy reads
-        // 8 bytes of the next row); on the generic kernel 10027 x 7424 took
-        // 199 us against 13.0 here, 1415 x 2304 20.9 against 6.3
-        return four ? launch_dma<23, 4, 2>(s, w, stride, rows, nblocks, x, y, 0, 1, nblocks % 2 != 0)
-                    : launch_dma<23, 8, 2>(s, w, stride, rows, nblocks, x, y, 0, 1, nblocks % 2 != 0);
+    if (encoding == 23 && nblocks % 2 == 0)
+        return four ? launch_dma<23, 4, 2>(s, w, stride, rows, nblocks, x, y, 0, 1)
+                    : launch_dma<23, 8, 2>(s, w, stride, rows, nblocks, x, y, 0, 1);
     return hipErrorInvalidValue;
 }
 

@@ -67,6 +67,9 @@ hipError_t launch_rows(hipStream_t s, uint32_t encoding, const uint8_t *w, uint6
                        uint64_t out_stride, uint32_t tokens);
 hipError_t launch_segments(hipStream_t s, const SegmentsArgs &args, const float *x);
 int segment_rows_per_wave();
+// One matrix on the merged kernel: F32 arithmetic, any row count.
+hipError_t launch_rows_f32(hipStream_t s, uint32_t encoding, const uint8_t *w, uint64_t stride, uint32_t rows,
+                           uint32_t columns, const float *x, float *y);
 hipError_t launch_argmax(hipStream_t s, const float *logits, uint64_t count, uint32_t *result);
 hipError_t launch_silu_mul(hipStream_t s, float *out, const float *up, uint32_t n);
 

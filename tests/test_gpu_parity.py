@@ -457,9 +457,10 @@ def test_silu_pair_large_runs_as_two_gemvs(backend, rows):
     (14, 20000, 2304), (23, 2, 256), (23, 17, 1280), (23, 1024, 4864), (23, 257, 17152), (23, 20000, 2304), (23, 1, 768),
 ])
 def test_last_row_and_row_ranges(backend, encoding, rows, columns):
-    """Q6_K and IQ4_XS rows that end mid-chunk: the last row has a workgroup
-    of its own (16-value groups against F32 x), beside 255 or 256 row ranges;
-    every row within the F32 bound, also with an infinity."""
+    """Q6_K and IQ4_XS rows that end mid-chunk: the last Q6_K row has a workgroup
+    of its own (16-value groups against F32 x), beside 255 or 256 row ranges,
+    and IQ4_XS rows run on the F32 row kernel; every row within the F32 bound,
+    also with an infinity."""
     import torch
     w = quantized(encoding, rows, columns, 61)
     m = nq.Matrix(encoding, rows, columns, to_gpu(w))
@@ -482,7 +483,7 @@ def test_last_row_and_row_ranges(backend, encoding, rows, columns):
 @pytest.mark.parametrize("encoding,columns,rows", [
     (8, 512, 4096), (8, 17408, 4112), (12, 256, 4112), (12, 17408, 4096), (13, 5120, 4368), (14, 2048, 4352),
     (14, 5120, 4096), (23, 512, 8208), (23, 4096, 4096),
-    (8, 4096, 2064), (12, 5120, 16), (13, 2048, 1024), (14, 2048, 272), (23, 512, 48), (23, 768, 32), (23, 3328, 4112),
+    (8, 4096, 2064), (8, 512, 48), (23, 3328, 4112),
 ])
 def test_silu_pair_equals_its_gemvs(backend, encoding, columns, rows):
     """The one-launch pair adds each row's sums as that matrix's own matvec
@@ -504,6 +505,67 @@ def test_silu_pair_equals_its_gemvs(backend, encoding, columns, rows):
         ok = torch.isfinite(want) & (want.abs() < 1e38)
         # expf, the quotient and the product round once or twice each
         assert ((out.double() - want)[ok].abs() <= 2e-6 * want[ok].abs() + 1e-37).all()
+
+
+def spread_input(encoding, rows, columns, seed):
+    """Weights and an x whose 32-value slices hold one value far above the
+    others, against a weight of zero (Q4_K, Q5_K) or of the smallest code
+    (IQ4_XS, in one slice): fixed point relative to the slice's maximum would
+    lose the others' low bits, F32 keeps them."""
+    w = quantized(encoding, rows, columns, seed)
+    b = w.reshape(rows, columns // 256, -1).copy()
+    x = gaussian(seed + 1, columns)
+    if encoding == 23:
+        x[0], x[32:] = 2.0**14, 0
+        b[:, 0, 8] = (b[:, 0, 8] & 0xf0) | 8
+    else:
+        x[::32] = 2.0**16
+        b[..., 2:4] = 0
+        b[..., (16 if encoding == 12 else 48) + 32 * np.arange(4)] = 0
+        if encoding == 13:
+            b[..., 16] = 0
+    return b.reshape(rows, -1), x
+
+
+@pytest.mark.parametrize("encoding,rows,columns", [(12, 16, 512), (12, 2048, 1280), (12, 4080, 256), (13, 16, 512),
+                                                   (13, 4080, 2304), (23, 48, 512), (23, 1024, 768), (23, 4080, 2048)])
+def test_small_pair_keeps_f32_activations(backend, encoding, rows, columns):
+    """SiLU pairs below 4096 rows run on F32 activations."""
+    import torch
+    gate, x = spread_input(encoding, rows, columns, 100)
+    up, _ = spread_input(encoding, rows, columns, 110)
+    out = torch.full((rows,), np.nan, device="cuda")
+    backend.matvec_segments([(nq.Matrix(encoding, rows, columns, to_gpu(a)), out) for a in (gate, up)], to_gpu(x),
+                            nq.SEGMENT_SILU_MUL_PAIR)
+    backend.sync()
+    dec = [orc.decode_matrix(encoding, a, rows, columns).astype(np.float64) for a in (gate, up)]
+    g, u = (d @ x.astype(np.float64) for d in dec)
+    eg, eu = (F32_K * (np.abs(d) @ np.abs(x).astype(np.float64)) for d in dec)
+    want = g / (1 + np.exp(-g)) * u
+    # the F32 bound of both products through silu(g) u (|silu'| <= 1.1)
+    bound = 1.1 * np.abs(u) * eg + (np.abs(g) + eg) * eu + 1e-6 * np.abs(want) + 1e-9
+    assert (np.abs(out.cpu().numpy() - want) <= bound).all()
+
+
+@pytest.mark.parametrize("calls", [[(23, 1415, 768)], [(23, 300, 17152)], [(23, 2, 256)], [(13, 272, 1280), (23, 48, 1280)],
+                                   [(12, 512, 2048), (13, 16, 2048), (23, 1024, 2048)]])
+def test_odd_rows_and_mixed_segments_keep_f32_activations(backend, calls):
+    """IQ4_XS rows of an odd block count, and plain segments of several
+    encodings with Q5_K or IQ4_XS among them."""
+    import torch
+    for lead in {c[0] for c in calls}:  # an x that spreads for each encoding in turn
+        data = [spread_input(e, r, c, 120 + i) for i, (e, r, c) in enumerate(calls)]
+        x = next(d[1] for d, c in zip(data, calls) if c[0] == lead)
+        outs = [torch.full((r,), np.nan, device="cuda") for _, r, _ in calls]
+        mats = [nq.Matrix(e, r, c, to_gpu(d[0])) for d, (e, r, c) in zip(data, calls)]
+        if len(calls) == 1:
+            backend.matvec(mats[0], to_gpu(x), outs[0])
+        else:
+            backend.matvec_segments(list(zip(mats, outs)), to_gpu(x), nq.SEGMENT_PLAIN)
+        backend.sync()
+        for (e, r, c), (w, _), o in zip(calls, data, outs):
+            dec, x64 = orc.decode_matrix(e, w, r, c).astype(np.float64), x.astype(np.float64)
+            assert (np.abs(o.cpu().numpy() - dec @ x64) <= F32_K * (np.abs(dec) @ np.abs(x64)) + 1e-9).all(), (lead, e)
 
 
 @pytest.mark.parametrize("encoding,columns,rows", [
