@@ -1289,6 +1289,9 @@ struct VSplit<13> {
 };
 
 constexpr int VF_MAX_WAVES = 16;
+// Two row groups per wave halve the x reads once there are enough rows to keep
+// 160 or more workgroups.
+constexpr uint32_t VF_TWO_GROUP_ROWS = 32 * 160;
 
 // RG row groups of 16 per wave: the x fragments of a block are loaded once
 // and feed RG MFMA chains, so a workgroup reads x once per 16*RG rows.
@@ -2290,9 +2293,7 @@ static hipError_t launch_verify_enc(hipStream_t s, const uint8_t *w, uint64_t st
     // measured best at K = 5120 (4 waves) and K = 17408 (14 waves).
     const uint32_t per_wave = std::max(5u, (nblocks + VF_MAX_WAVES - 1) / VF_MAX_WAVES);
     const uint32_t waves = (nblocks + per_wave - 1) / per_wave;
-    // Two row groups per wave halve the x reads once there are enough rows
-    // to keep 160 or more workgroups.
-    if (rows >= 32u * 160)
+    if (rows >= VF_TWO_GROUP_ROWS)
         return launch_verify_rg<ENC, 2>(s, w, stride, rows, nblocks, waves, x, x_f16, in_stride, y, out_stride, tokens);
     return launch_verify_rg<ENC, 1>(s, w, stride, rows, nblocks, waves, x, x_f16, in_stride, y, out_stride, tokens);
 }
@@ -2366,6 +2367,28 @@ static float prefill_cost(uint32_t rows, uint32_t columns, uint32_t tokens, uint
            0.4f * (float)tail * splits * (PF_BM * PF_BN * 4e-6f);
 }
 
+// Whether 4 to 16 f16 tokens of Q8_0, Q6_K or IQ4_XS run faster on the panel
+// tile, by its plan `p`, than on the register verify tile. The verify tile takes
+// a + (b + c tokens) us per 256-column block of 16 rows on the busiest CU, so it
+// wins where its row groups fill the CUs in whole rounds (4096 rows: one each);
+// the panel model is low by the last two factors for whole and split tiles at
+// these tokens. Fitted to 172 timings each (43 matrices of 2^25 weights and more, 4 to
+// 16 tokens): the choice takes 1.004 (Q8_0), 1.009 (Q6_K) and 1.006 (IQ4_XS)
+// of the better tile's time on average and 1.15 at most over the verify tile's,
+// where the panel tile for all took up to 1.44, 1.37 and 1.72 (IQ4_XS 4096 x
+// 9216 at 4 tokens 18.7 us against 10.8).
+static bool panel_beats_verify(uint32_t encoding, uint32_t rows, uint32_t columns, uint32_t tokens,
+                               const PanelPlan &p) {
+    struct {
+        float a, b, c, whole, split;
+    } const k = encoding == 8    ? decltype(k){0.4f, 0.355f, 0.011f, 1.15f, 0.9f}
+                : encoding == 14 ? decltype(k){3.9f, 0.247f, 0.0053f, 1.25f, 1.05f}
+                                 : decltype(k){6.2f, 0.129f, 0.0095f, 1.25f, 1.1f};
+    const uint32_t groups = rows >= VF_TWO_GROUP_ROWS ? 2 : 1, wgs = (rows + 16 * groups - 1) / (16 * groups);
+    const float blocks = (float)((wgs + 255) / 256 * groups) * (float)(columns / 256);
+    return p.cost * (p.splits > 1 ? k.split : k.whole) < k.a + blocks * (k.b + k.c * (float)tokens);
+}
+
 // At most this much f16 copy of F32 activations at a time (bytes).
 constexpr uint64_t X16_BYTES = 256ull << 20;
 
@@ -2373,10 +2396,12 @@ constexpr uint64_t X16_BYTES = 256ull << 20;
 //  - Q4_K / Q5_K up to VF_PASS_MAX tokens keep the streamed verify tile, whose
 //    products are exact (the panel tile rounds weights to f16).
 //  - Otherwise the panel tile, from 17 tokens, and from 4 for matrices of at
-//    least 2^25 weights: Q6_K 5120 x 17408 at 4 / 16 tokens 28 / 29 us against
-//    38 / 44 on the register verify tile, 5120 x 6144 15.8 / 16 against
-//    15.8 / 18, 4096 x 4096 11-15 against 7-10 (it needs the split and its
-//    reduction there).
+//    least 2^25 weights: with F32 activations, which the register verify tile
+//    reads and rounds once per 16 or 32 rows, always (Q6_K 5120 x 17408 at 4 / 16
+//    tokens 30 / 32 us against 46 / 61, 8192 x 4096 18 / 18 against 21 / 23,
+//    IQ4_XS 8192 x 4096 16 / 17 against 19 / 21, Q8_0 20 / 21 against 24 / 27; of
+//    516 timings one lost over 5 %: IQ4_XS 4096 x 9216 at 4 tokens, 8 %),
+//    with f16 ones where panel_beats_verify.
 //  - Q8_0 may run on the prefill tile where that is predicted faster: its raw
 //    bytes are twice the others', and the panel tile reads them once per 128 or
 //    256 tokens of every row tile through LDS (17408 x 5120 at 4096 tokens 779
@@ -2426,6 +2451,7 @@ void plan_tile(uint32_t encoding, uint32_t rows, uint32_t columns, uint32_t toke
         (short_chunk == 0 ||
          panel_plan(encoding, rows, columns, short_chunk, stride, row_stride, t->panel.work_floats, &t->last))) {
         const bool both = !small && t->route == TilePlan::PREFILL && encoding == 8;
+        if (small && x_f16 && !panel_beats_verify(encoding, rows, columns, tokens, t->panel)) return;
         if (!both ||
             t->panel.cost < 0.92f * prefill_cost(rows, columns, chunk, std::min(max_floats - copy, split_max))) {
             t->route = TilePlan::PANEL;
@@ -2450,6 +2476,15 @@ void plan_tile(uint32_t encoding, uint32_t rows, uint32_t columns, uint32_t toke
     prefill_split_plan(tiles, columns, compute_units(), std::min(max_floats - t->copy, split_max) / (PF_BM * PF_BN),
                        &full, &tail, &splits);
     t->floats = (uint64_t)tail * splits * PF_BM * PF_BN + t->copy;
+}
+
+// The route plan_tile takes with any workspace, for checks on the host.
+extern "C" int nuq_tile_route(uint32_t encoding, uint32_t rows, uint32_t columns, uint32_t tokens, uint32_t x_f16) {
+    Layout l;
+    if (!layout_of(encoding, &l)) return -1;
+    TilePlan t;
+    plan_tile(encoding, rows, columns, tokens, x_f16, (uint64_t)columns / l.elements * l.bytes, columns, UINT64_MAX, &t);
+    return t.route;
 }
 
 static hipError_t launch_verify(hipStream_t s, uint32_t encoding, const uint8_t *w, uint64_t stride, uint32_t rows,

@@ -157,16 +157,16 @@ bool panel_plan(uint32_t encoding, uint32_t rows, uint32_t columns, uint32_t tok
 }
 
 // The plan as plain numbers (shape, full, tail, splits, partial floats, then the
-// shape's tokens and rows of a tile and K sets), for checks on the host; 0 when
-// the tile does not take the product.
+// shape's tokens and rows of a tile, its K sets and the predicted ns), for
+// checks on the host; 0 when the tile does not take the product.
 extern "C" int nuq_panel_plan(uint32_t encoding, uint32_t rows, uint32_t columns, uint32_t tokens, uint64_t stride,
-                              uint64_t in_stride, uint64_t max_floats, uint64_t out[8]) {
+                              uint64_t in_stride, uint64_t max_floats, uint64_t out[9]) {
     PanelPlan p;
     if (!panel_plan(encoding, rows, columns, tokens, stride, in_stride, max_floats, &p)) return 0;
     const PanelShape &s = PANEL_SHAPES[p.shape];
-    const uint64_t v[8] = {(uint64_t)p.shape, p.full, p.tail, p.splits, p.work_floats,
-                           32ull * s.tg, 32ull * s.rg * s.wr, s.wk};
-    std::copy(v, v + 8, out);
+    const uint64_t v[9] = {(uint64_t)p.shape, p.full, p.tail, p.splits, p.work_floats,
+                           32ull * s.tg, 32ull * s.rg * s.wr, s.wk, (uint64_t)(p.cost * 1e3f)};
+    std::copy(v, v + 9, out);
     return 1;
 }
 

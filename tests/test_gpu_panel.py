@@ -309,3 +309,22 @@ def test_one_block_rows_in_parts(backend, encoding):
     xr = x[check].half().float().cpu().numpy()
     check_close(y[check].cpu().numpy(), orc.matmul(encoding, rows, columns, w, xr), mass(encoding, w, rows, columns, xr),
                 F16_K, f"panel-one-block {encoding} in parts")
+
+
+@pytest.mark.parametrize("encoding", [8, 14, 23])
+@pytest.mark.parametrize("tokens", [4, 7, 16])
+def test_few_tokens_on_a_large_matrix(backend, encoding, tokens):
+    """4 to 16 tokens on 2^25 weights and more run on the panel tile."""
+    import torch
+    rows, columns = 8 * 129, 32768
+    print(f"[panel] enc {encoding} {rows}x{columns} tokens {tokens}", flush=True)
+    part = nq.quantize(encoding, gaussian(91, (129, columns), 0.02))
+    m = nq.Matrix(encoding, rows, columns, to_gpu(np.tile(part, (8, 1))))
+    x = to_gpu(gaussian(92, (tokens, columns)))
+    xr = x.half().float().cpu().numpy()
+    want, ms = (np.tile(a, 8) for a in (orc.matmul(encoding, 129, columns, part, xr), mass(encoding, part, 129, columns, xr)))
+    for xg in (x, x.half()):
+        y = torch.full((tokens, rows), float("nan"), device="cuda")
+        backend.matmul(m, xg, columns, y, rows, tokens)
+        backend.sync()
+        check_close(y.cpu().numpy(), want, ms, F16_K, f"panel-few {encoding} tokens {tokens}")

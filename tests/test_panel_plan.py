@@ -12,8 +12,8 @@ import nuclis_amd as nq
 def plan(encoding, rows, columns, tokens, max_floats, in_stride=None):
     f = nq.lib().nuq_panel_plan
     u32, u64 = ctypes.c_uint32, ctypes.c_uint64
-    f.argtypes = [u32, u32, u32, u32, u64, u64, u64, u64 * 8]
-    out = (u64 * 8)()
+    f.argtypes = [u32, u32, u32, u32, u64, u64, u64, u64 * 9]
+    out = (u64 * 9)()
     ok = f(encoding, rows, columns, tokens, nq.row_bytes(encoding, columns), in_stride or columns, max_floats, out)
     return list(out) if ok else None
 
@@ -22,7 +22,8 @@ def check(encoding, rows, columns, tokens, max_floats):
     where = f"enc {encoding} {rows}x{columns} tokens {tokens} workspace {max_floats}"
     p = plan(encoding, rows, columns, tokens, max_floats)
     assert p is not None, where
-    shape, full, tail, splits, floats, bm, bn, sets = p
+    shape, full, tail, splits, floats, bm, bn, sets, ns = p
+    assert ns > 0, where
     nb = columns // 256
     assert full + tail == -(-tokens // bm) * -(-rows // bn), where
     # every wave set of every split has a 256-column block
@@ -48,6 +49,72 @@ def test_refuses_what_the_tile_cannot_address():
     """Copies use 32-bit offsets within a tile; 64-column remainders and other
     encodings have no panel form."""
     assert plan(12, 64, 320, 100, 0) is None
-    assert nq.lib().nuq_panel_plan(0, 64, 256, 100, 144, 256, 0, (ctypes.c_uint64 * 8)()) == 0
+    assert nq.lib().nuq_panel_plan(0, 64, 256, 100, 144, 256, 0, (ctypes.c_uint64 * 9)()) == 0
     assert plan(12, 64, 256, 100, 0, in_stride=1 << 23) is None
     assert plan(12, 64, 256, 100, 0, in_stride=1 << 22) is not None
+
+
+# encoding, rows, columns, tokens, us on the register verify tile, us on the
+# panel tile: f16 activations, measured on MI355X
+MEASURED = [
+    (8, 4096, 9216, 4, 13.9, 18.4), (8, 4096, 9216, 16, 23.3, 19.1),
+    (8, 8192, 4096, 4, 16.7, 17.8), (8, 8192, 4096, 16, 20.3, 18.6),
+    (8, 4096, 14336, 4, 26.3, 22.9), (8, 4096, 14336, 16, 40.1, 23.2),
+    (8, 5120, 17408, 4, 55.4, 38.3), (8, 5120, 17408, 16, 76.2, 40.0),
+    (8, 17408, 5120, 4, 48.6, 38.1), (8, 17408, 5120, 16, 66.8, 40.2),
+    (8, 1024, 32768, 4, 56.0, 19.2), (8, 1024, 32768, 16, 82.7, 19.9),
+    (8, 16384, 2048, 4, 17.7, 15.6), (8, 16384, 2048, 16, 18.9, 16.0),
+    (8, 28672, 8192, 4, 129.7, 86.5), (8, 28672, 8192, 16, 174.6, 86.9),
+    (8, 7168, 7168, 4, 21.0, 22.0), (8, 7168, 7168, 16, 26.0, 22.5),
+    (8, 12288, 6144, 4, 39.4, 28.6), (8, 12288, 6144, 16, 50.0, 30.3),
+    (14, 4096, 9216, 4, 14.3, 19.5), (14, 4096, 9216, 16, 18.1, 17.5),
+    (14, 8192, 4096, 4, 12.4, 15.5), (14, 8192, 4096, 16, 13.5, 16.2),
+    (14, 4096, 14336, 4, 18.8, 21.1), (14, 4096, 14336, 16, 25.0, 21.6),
+    (14, 5120, 17408, 4, 36.9, 28.2), (14, 5120, 17408, 16, 43.4, 29.1),
+    (14, 17408, 5120, 4, 33.9, 27.3), (14, 17408, 5120, 16, 40.0, 28.4),
+    (14, 1024, 32768, 4, 49.9, 16.8), (14, 1024, 32768, 16, 65.9, 17.4),
+    (14, 16384, 2048, 4, 14.4, 12.8), (14, 16384, 2048, 16, 14.8, 13.2),
+    (14, 28672, 8192, 4, 74.3, 64.7), (14, 28672, 8192, 16, 97.8, 68.0),
+    (14, 7168, 7168, 4, 17.9, 19.4), (14, 7168, 7168, 16, 20.3, 20.3),
+    (14, 12288, 6144, 4, 28.5, 23.6), (14, 12288, 6144, 16, 33.7, 26.3),
+    (23, 4096, 9216, 4, 10.8, 18.7), (23, 4096, 9216, 16, 17.6, 16.6),
+    (23, 8192, 4096, 4, 12.0, 13.7), (23, 8192, 4096, 16, 17.4, 15.0),
+    (23, 4096, 14336, 4, 13.8, 20.5), (23, 4096, 14336, 16, 27.3, 21.1),
+    (23, 5120, 17408, 4, 27.6, 27.6), (23, 5120, 17408, 16, 38.5, 28.6),
+    (23, 17408, 5120, 4, 26.0, 27.4), (23, 17408, 5120, 16, 36.4, 29.0),
+    (23, 1024, 32768, 4, 27.6, 15.1), (23, 1024, 32768, 16, 50.6, 15.8),
+    (23, 16384, 2048, 4, 14.7, 11.2), (23, 16384, 2048, 16, 16.6, 11.6),
+    (23, 28672, 8192, 4, 59.0, 59.8), (23, 28672, 8192, 16, 89.3, 60.4),
+    (23, 7168, 7168, 4, 17.7, 19.4), (23, 7168, 7168, 16, 21.9, 20.5),
+    (23, 12288, 6144, 4, 23.5, 23.5), (23, 12288, 6144, 16, 30.8, 23.8),
+]
+VERIFY, PANEL = 0, 1  # TilePlan::Route
+
+
+def route(encoding, rows, columns, tokens, x_f16):
+    f = nq.lib().nuq_tile_route
+    f.argtypes = [ctypes.c_uint32] * 5
+    return f(encoding, rows, columns, tokens, x_f16)
+
+
+def test_few_tokens_take_the_faster_tile():
+    """4 to 16 f16 tokens on large matrices: the predicted choice is never much
+    slower than the other tile."""
+    for encoding, rows, columns, tokens, verify, panel in MEASURED:
+        r = route(encoding, rows, columns, tokens, 1)
+        assert r in (VERIFY, PANEL)
+        chosen = panel if r == PANEL else verify
+        assert chosen <= 1.16 * min(verify, panel), (encoding, rows, columns, tokens, r, verify, panel)
+
+
+@pytest.mark.parametrize("encoding", [8, 14, 23])
+def test_few_f32_tokens_and_small_matrices(encoding):
+    """F32 activations take the panel tile from 4 tokens and 2^25 weights, the
+    verify tile below."""
+    for tokens in (4, 9, 16):
+        assert route(encoding, 4096, 8192, tokens, 0) == PANEL
+        assert route(encoding, 4088, 8192, tokens, 0) == route(encoding, 4088, 8192, tokens, 1) == VERIFY
+    assert route(encoding, 1 << 15, 1 << 15, 3, 0) == route(encoding, 1 << 15, 1 << 15, 3, 1) == VERIFY
+    for e in (12, 13):
+        assert route(e, 5120, 17408, 16, 0) == route(e, 5120, 17408, 48, 1) == VERIFY
+        assert route(e, 5120, 17408, 49, 0) == route(e, 5120, 17408, 49, 1) == PANEL
