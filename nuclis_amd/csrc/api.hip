@@ -35,9 +35,10 @@ struct nuq_context {
     bool generic_only = false;
     std::string last_error;
     uint32_t *argmax_buf = nullptr;  // device: {index, nonfinite flag}
-    // F32 workspace of the verify K ranges, the prefill split partials and
-    // the SiLU pair's second GEMV: allocated on the first call that wants it
-    // and grown in whole 256 x 256 tiles (ensure_workspace)
+    // F32 workspace of the verify K ranges, the split tiles' partial sums, the
+    // f16 copy of F32 activations and the second GEMV of a SiLU pair of two
+    // encodings: allocated on the first call that wants it and grown in whole
+    // 256 x 256 tiles (ensure_workspace)
     nuq::SplitScratch split{nullptr, 0};
     // The current workspace was handed to a launch recorded into a graph:
     // on growth it is kept (the graph may replay) rather than freed.
@@ -94,7 +95,11 @@ bool capture_active(hipStream_t stream) {
 }
 
 // Grows the context workspace to at least `floats` F32 values (whole 256 x
-// 256 tiles). Returns false, leaving it as it was, when the allocation fails
+// 256 tiles), and with `headroom` to a power of two of them from 4 MiB to 512
+// (the most the tiles' plans ask for): the f16 copy of F32 activations grows
+// with the prompt, and an allocation, a wait for the stream and a free on each
+// prompt longer than all before would cost more than the product; so a context
+// pays at most eight of them. Returns false, leaving it as it was, when the allocation fails
 // or a graph capture is active (an allocation cannot be captured): the
 // caller's route then takes its no-workspace form, or fewer splits of the
 // workspace it has, which compute the same products. A call made while its
@@ -103,8 +108,8 @@ bool capture_active(hipStream_t stream) {
 // it), and otherwise frees it once the context's stream has finished with
 // it (a stream change orders the new stream after the old, so that wait
 // covers every call of the context).
-bool ensure_workspace(nuq_context *ctx, uint64_t floats) {
-    constexpr uint64_t TILE = 256 * 256;
+bool ensure_workspace(nuq_context *ctx, uint64_t floats, bool headroom = true) {
+    constexpr uint64_t TILE = 256 * 256, LEAST = 16, MOST = 2048;
     if (floats == 0) return true;
     const uint64_t tiles = (floats + TILE - 1) / TILE;
     if (capture_active(ctx->stream)) {
@@ -114,9 +119,18 @@ bool ensure_workspace(nuq_context *ctx, uint64_t floats) {
     if (tiles <= ctx->split.tiles) return true;
     if (tiles > 0xffffffffull) return false;
     float *p = nullptr;
-    if (hipMalloc((void **)&p, tiles * TILE * sizeof(float)) != hipSuccess) {
+    uint64_t target = LEAST;
+    while (target < tiles) target *= 2;
+    if (!headroom || target > MOST) target = tiles;
+    if (hipMalloc((void **)&p, target * TILE * sizeof(float)) != hipSuccess) {
         (void)hipGetLastError();
-        return false;
+        p = nullptr;
+        if (target != tiles && hipMalloc((void **)&p, tiles * TILE * sizeof(float)) != hipSuccess) {
+            (void)hipGetLastError();
+            p = nullptr;
+        }
+        if (!p) return false;
+        target = tiles;
     }
     if (ctx->split.work) {
         if (ctx->split_captured) {
@@ -127,7 +141,7 @@ bool ensure_workspace(nuq_context *ctx, uint64_t floats) {
         }
     }
     ctx->split.work = p;
-    ctx->split.tiles = (uint32_t)tiles;
+    ctx->split.tiles = (uint32_t)target;
     ctx->split_captured = false;
     return true;
 }
@@ -421,7 +435,7 @@ int nuq_set_stream(nuq_context *ctx, void *stream) {
 int nuq_reserve_workspace(nuq_context *ctx, uint64_t bytes) {
     if (!ctx) return NUQ_INVALID_ARGUMENT;
     (void)hipSetDevice(ctx->device);
-    if (!ensure_workspace(ctx, (bytes + sizeof(float) - 1) / sizeof(float)))
+    if (!ensure_workspace(ctx, (bytes + sizeof(float) - 1) / sizeof(float), false))
         return fail(ctx, NUQ_DEVICE_ERROR, "workspace of %llu bytes could not be allocated (or the stream is capturing)",
                     (unsigned long long)bytes);
     return NUQ_OK;

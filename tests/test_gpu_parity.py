@@ -671,6 +671,31 @@ def test_workspace_is_allocated_lazily():
         b.close()
 
 
+def test_growing_prompts_seldom_grow_the_workspace():
+    """F32 prompts, each longer than all before: the workspace (the f16 copy of
+    the activations among it) grows by powers of two, and a reserved size is
+    taken as it is."""
+    import torch
+    b = nq.Backend(0)
+    try:
+        rows, columns = 64, 8192
+        m = nq.Matrix(14, rows, columns, to_gpu(quantized(14, rows, columns, 144)))
+        x = torch.randn((2048, columns), device="cuda")
+        y = torch.empty((2048, rows), device="cuda")
+        sizes = []
+        for tokens in range(64, 2049, 64):
+            b.matmul(m, x, columns, y, rows, tokens)
+            sizes.append(b.workspace_bytes())
+        b.sync()
+        assert sizes == sorted(sizes) and sizes[-1] >= 2048 * columns * 2
+        # 4, 8, ... 64 MiB
+        assert len(set(sizes)) <= 5, sizes
+        b.reserve_workspace(100 << 20)
+        assert b.workspace_bytes() == 100 << 20
+    finally:
+        b.close()
+
+
 def test_captured_workspace_survives_growth():
     """A graph captured with the context's workspace (the verify tile's K
     ranges) still replays correctly after a later eager call has grown the
