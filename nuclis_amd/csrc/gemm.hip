@@ -2355,14 +2355,14 @@ uint64_t verify_workspace_floats(uint32_t encoding, uint32_t rows, uint32_t colu
 }
 
 // Predicted time (us) of Q8_0 on the prefill tile with f16 activations: 3.6 us
-// a round of 256 tiles, 8.54 us a 256-column block of a round, 0.4 us per MB of
+// a round of a tile per CU, 8.54 us a 256-column block of a round, 0.4 us per MB of
 // split partial sums. Fitted to the times from 64 to 4096 tokens on 17408 x
 // 5120, 5120 x 17408 and 4096 x 4096 (6 % rms).
-static float prefill_cost(uint32_t rows, uint32_t columns, uint32_t tokens, uint64_t max_floats) {
+static float prefill_cost(uint32_t rows, uint32_t columns, uint32_t tokens, uint64_t max_floats, uint32_t cus) {
     const uint32_t tiles = ((tokens + PF_BM - 1) / PF_BM) * ((rows + PF_BN - 1) / PF_BN), nb = columns / 256;
     uint32_t full, tail, splits;
-    prefill_split_plan(tiles, columns, 256, max_floats / (PF_BM * PF_BN), &full, &tail, &splits);
-    const uint32_t r1 = (full + 255) / 256, r2 = (tail * splits + 255) / 256;
+    prefill_split_plan(tiles, columns, cus, max_floats / (PF_BM * PF_BN), &full, &tail, &splits);
+    const uint32_t r1 = (full + cus - 1) / cus, r2 = (tail * splits + cus - 1) / cus;
     return 3.6f * (r1 + r2) + 8.54f * (r1 * nb + r2 * ((nb + splits - 1) / splits)) +
            0.4f * (float)tail * splits * (PF_BM * PF_BN * 4e-6f);
 }
@@ -2378,14 +2378,14 @@ static float prefill_cost(uint32_t rows, uint32_t columns, uint32_t tokens, uint
 // where the panel tile for all took up to 1.44, 1.37 and 1.72 (IQ4_XS 4096 x
 // 9216 at 4 tokens 18.7 us against 10.8).
 static bool panel_beats_verify(uint32_t encoding, uint32_t rows, uint32_t columns, uint32_t tokens,
-                               const PanelPlan &p) {
+                               const PanelPlan &p, uint32_t cus) {
     struct {
         float a, b, c, whole, split;
     } const k = encoding == 8    ? decltype(k){0.4f, 0.355f, 0.011f, 1.15f, 0.9f}
                 : encoding == 14 ? decltype(k){3.9f, 0.247f, 0.0053f, 1.25f, 1.05f}
                                  : decltype(k){6.2f, 0.129f, 0.0095f, 1.25f, 1.1f};
     const uint32_t groups = rows >= VF_TWO_GROUP_ROWS ? 2 : 1, wgs = (rows + 16 * groups - 1) / (16 * groups);
-    const float blocks = (float)((wgs + 255) / 256 * groups) * (float)(columns / 256);
+    const float blocks = (float)((wgs + cus - 1) / cus * groups) * (float)(columns / 256);
     return p.cost * (p.splits > 1 ? k.split : k.whole) < k.a + blocks * (k.b + k.c * (float)tokens);
 }
 
@@ -2441,19 +2441,20 @@ void plan_tile(uint32_t encoding, uint32_t rows, uint32_t columns, uint32_t toke
         copy = ((uint64_t)chunk * columns + 1) / 2;
     }
     const uint64_t row_stride = x_f16 ? in_stride : columns;
+    const uint32_t cus = compute_units();
     const uint64_t split_max = (uint64_t)split_scratch_tiles() * PF_BM * PF_BN;
     const bool room = chunk != 0 && copy <= max_floats;
     // (a shorter last chunk is planned here too, within the others' partials, so
     // that none can be refused once another has run)
     const uint32_t short_chunk = room ? tokens % chunk : 0;
     if (room && panel_plan(encoding, rows, columns, chunk, stride, row_stride, std::min(max_floats - copy, split_max),
-                           &t->panel) &&
+                           cus, &t->panel) &&
         (short_chunk == 0 ||
-         panel_plan(encoding, rows, columns, short_chunk, stride, row_stride, t->panel.work_floats, &t->last))) {
+         panel_plan(encoding, rows, columns, short_chunk, stride, row_stride, t->panel.work_floats, cus, &t->last))) {
         const bool both = !small && t->route == TilePlan::PREFILL && encoding == 8;
-        if (small && x_f16 && !panel_beats_verify(encoding, rows, columns, tokens, t->panel)) return;
+        if (small && x_f16 && !panel_beats_verify(encoding, rows, columns, tokens, t->panel, cus)) return;
         if (!both ||
-            t->panel.cost < 0.92f * prefill_cost(rows, columns, chunk, std::min(max_floats - copy, split_max))) {
+            t->panel.cost < 0.92f * prefill_cost(rows, columns, chunk, std::min(max_floats - copy, split_max), cus)) {
             t->route = TilePlan::PANEL;
             t->chunk = chunk;
             t->copy = copy;
@@ -2473,7 +2474,7 @@ void plan_tile(uint32_t encoding, uint32_t rows, uint32_t columns, uint32_t toke
     }
     const uint32_t tiles = ((t->chunk + PF_BM - 1) / PF_BM) * ((rows + PF_BN - 1) / PF_BN);
     uint32_t full, tail, splits;
-    prefill_split_plan(tiles, columns, compute_units(), std::min(max_floats - t->copy, split_max) / (PF_BM * PF_BN),
+    prefill_split_plan(tiles, columns, cus, std::min(max_floats - t->copy, split_max) / (PF_BM * PF_BN),
                        &full, &tail, &splits);
     t->floats = (uint64_t)tail * splits * PF_BM * PF_BN + t->copy;
 }
@@ -2528,10 +2529,10 @@ hipError_t launch_tile(hipStream_t s, uint32_t encoding, const uint8_t *w, uint6
         }
         return hipSuccess;
     }
-    if (plan.route == TilePlan::TILE || (plan.route == TilePlan::PREFILL && plan.copy == 0)) {
-        if (plan.route == TilePlan::PREFILL)
-            return launch_prefill_any(s, encoding, w, stride, rows, columns, x, x_f16, in_stride, y, out_stride, tokens,
-                                      scratch);
+    if (plan.route == TilePlan::PREFILL && plan.copy == 0)
+        return launch_prefill_any(s, encoding, w, stride, rows, columns, x, x_f16, in_stride, y, out_stride, tokens,
+                                  scratch);
+    if (plan.route == TilePlan::TILE) {
         switch (encoding) {
         case 12: return launch_tile_enc<12>(s, w, stride, rows, columns, x, x_f16, in_stride, y, out_stride, tokens);
         case 13: return launch_tile_enc<13>(s, w, stride, rows, columns, x, x_f16, in_stride, y, out_stride, tokens);

@@ -42,10 +42,10 @@ struct PanelArgs {
     uint32_t tokens;
 };
 
-// The fastest plan by the cost model with at most max_floats of workspace;
-// false when the tile does not take the product.
+// The fastest plan by the cost model on `cus` compute units with at most
+// max_floats of workspace; false when the tile does not take the product.
 bool panel_plan(uint32_t encoding, uint32_t rows, uint32_t columns, uint32_t tokens, uint64_t stride,
-                uint64_t in_stride, uint64_t max_floats, PanelPlan *plan);
+                uint64_t in_stride, uint64_t max_floats, uint32_t cus, PanelPlan *plan);
 hipError_t launch_panel(hipStream_t s, uint32_t encoding, const PanelArgs &a, const PanelPlan &p, float *work);
 // f32 rows of `columns` values, `in_stride` apart, to packed f16 rows.
 hipError_t launch_to_f16(hipStream_t s, const float *x, uint64_t in_stride, uint32_t columns, uint32_t tokens,

@@ -94,17 +94,17 @@ static int encoding_index(uint32_t encoding) {
 }
 
 // `count` workgroups of `blocks` 256-column blocks each
-static float rounds_cost(const PanelCost &k, uint32_t wk, uint32_t count, uint32_t blocks) {
+static float rounds_cost(const PanelCost &k, uint32_t cus, uint32_t wk, uint32_t count, uint32_t blocks) {
     if (count == 0) return 0.f;
-    const uint32_t cap = 256 * k.occ, whole = count / cap, rest = count % cap;
+    const uint32_t cap = cus * k.occ, whole = count / cap, rest = count % cap;
     const float n = (float)((blocks + wk - 1) / wk);
     float t = (float)whole * (k.a + n * (k.b + k.c * (float)(k.occ - 1)));
-    if (rest) t += k.a + n * (k.b + k.c * (float)((rest + 255) / 256 - 1));
+    if (rest) t += k.a + n * (k.b + k.c * (float)((rest + cus - 1) / cus - 1));
     return t;
 }
 
 bool panel_plan(uint32_t encoding, uint32_t rows, uint32_t columns, uint32_t tokens, uint64_t stride,
-                uint64_t in_stride, uint64_t max_floats, PanelPlan *plan) {
+                uint64_t in_stride, uint64_t max_floats, uint32_t cus, PanelPlan *plan) {
     const int e = encoding_index(encoding);
     if (e < 0 || columns % 256 != 0 || tokens == 0) return false;
     // copies use 32-bit offsets within a tile (at most 256 rows or tokens)
@@ -121,7 +121,7 @@ bool panel_plan(uint32_t encoding, uint32_t rows, uint32_t columns, uint32_t tok
         const PanelShape &s = PANEL_SHAPES[i];
         const PanelCost &k = PANEL_COST[e][i];
         if (s.tg > widest || (s.tg < 4 && groups > 2u * s.tg) || nb < s.wk) continue;
-        const uint32_t bm = 32 * s.tg, bn = 32 * s.rg * s.wr, cap = 256 * k.occ;
+        const uint32_t bm = 32 * s.tg, bn = 32 * s.rg * s.wr, cap = cus * k.occ;
         const uint64_t tiles64 = (uint64_t)((tokens + bm - 1) / bm) * ((rows + bn - 1) / bn);
         if (tiles64 > 0x7fffffffu / 32) continue;
         const uint32_t tiles = (uint32_t)tiles64;
@@ -130,11 +130,11 @@ bool panel_plan(uint32_t encoding, uint32_t rows, uint32_t columns, uint32_t tok
             if (floats > max_floats) return;
             float t;
             if (splits == 1) {
-                t = rounds_cost(k, s.wk, tiles, nb);
+                t = rounds_cost(k, cus, s.wk, tiles, nb);
             } else {
                 // the reduction moves the partial sums of real tokens and rows once in, and the results out
                 const float sums = tail == tiles ? std::min((float)tail * bm * bn, (float)tokens * rows) : (float)tail * bm * bn;
-                t = rounds_cost(k, s.wk, tiles - tail, nb) + rounds_cost(k, s.wk, tail * splits, (nb + splits - 1) / splits) +
+                t = rounds_cost(k, cus, s.wk, tiles - tail, nb) + rounds_cost(k, cus, s.wk, tail * splits, (nb + splits - 1) / splits) +
                     k.r0 + k.r1 * 4e-6f * sums * ((float)splits + 0.5f);
             }
             if (found && t >= plan->cost) return;
@@ -144,7 +144,7 @@ bool panel_plan(uint32_t encoding, uint32_t rows, uint32_t columns, uint32_t tok
         consider(0, 1);
         // all tiles split, to one to four workgroups per CU
         if (tiles < 2 * cap)
-            for (uint32_t u = 256; u <= 1024; u += 256)
+            for (uint32_t u = cus; u <= 4 * cus; u += cus)
                 for (uint32_t r = 0; r < 2; ++r) {
                     const uint32_t sp = r ? (u + tiles - 1) / tiles : u / tiles;
                     if (sp > 1 && sp <= 24 && sp * s.wk <= nb) consider(tiles, sp);
@@ -160,9 +160,9 @@ bool panel_plan(uint32_t encoding, uint32_t rows, uint32_t columns, uint32_t tok
 // shape's tokens and rows of a tile, its K sets and the predicted ns), for
 // checks on the host; 0 when the tile does not take the product.
 extern "C" int nuq_panel_plan(uint32_t encoding, uint32_t rows, uint32_t columns, uint32_t tokens, uint64_t stride,
-                              uint64_t in_stride, uint64_t max_floats, uint64_t out[9]) {
+                              uint64_t in_stride, uint64_t max_floats, uint32_t cus, uint64_t out[9]) {
     PanelPlan p;
-    if (!panel_plan(encoding, rows, columns, tokens, stride, in_stride, max_floats, &p)) return 0;
+    if (!panel_plan(encoding, rows, columns, tokens, stride, in_stride, max_floats, cus, &p)) return 0;
     const PanelShape &s = PANEL_SHAPES[p.shape];
     const uint64_t v[9] = {(uint64_t)p.shape, p.full, p.tail, p.splits, p.work_floats,
                            32ull * s.tg, 32ull * s.rg * s.wr, s.wk, (uint64_t)(p.cost * 1e3f)};

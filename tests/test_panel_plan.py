@@ -1,6 +1,6 @@
 """The panel tile's planner on the host: every product the tile's shape rule
-admits has a plan, with and without workspace, and the plan covers the product.
-No GPU is used (the cost model then assumes 256 compute units)."""
+admits has a plan, with and without workspace, and the plan covers the product;
+the routes beside it. No GPU is used."""
 import ctypes
 import random
 
@@ -9,12 +9,12 @@ import pytest
 import nuclis_amd as nq
 
 
-def plan(encoding, rows, columns, tokens, max_floats, in_stride=None):
+def plan(encoding, rows, columns, tokens, max_floats, in_stride=None, cus=256):
     f = nq.lib().nuq_panel_plan
     u32, u64 = ctypes.c_uint32, ctypes.c_uint64
-    f.argtypes = [u32, u32, u32, u32, u64, u64, u64, u64 * 9]
+    f.argtypes = [u32, u32, u32, u32, u64, u64, u64, u32, u64 * 9]
     out = (u64 * 9)()
-    ok = f(encoding, rows, columns, tokens, nq.row_bytes(encoding, columns), in_stride or columns, max_floats, out)
+    ok = f(encoding, rows, columns, tokens, nq.row_bytes(encoding, columns), in_stride or columns, max_floats, cus, out)
     return list(out) if ok else None
 
 
@@ -45,11 +45,25 @@ def test_every_product_has_a_plan(encoding):
               rng.choice([0, 1 << 20, 1 << 26]))
 
 
+@pytest.mark.parametrize("cus", [256, 128, 304])
+def test_split_tails_leave_whole_rounds(cus):
+    """Where only the tiles of a partial last round are split, the whole tiles
+    fill the rounds of the CUs that are there."""
+    seen = 0
+    for rows in range(1024, 17409, 1024):
+        for tokens in range(256, 4097, 256):
+            p = plan(12, rows, 5120, tokens, 1 << 26, cus=cus)
+            if p[1] and p[2]:
+                seen += 1
+                assert p[1] % cus == 0, (rows, tokens, p)
+    assert seen
+
+
 def test_refuses_what_the_tile_cannot_address():
     """Copies use 32-bit offsets within a tile; 64-column remainders and other
     encodings have no panel form."""
     assert plan(12, 64, 320, 100, 0) is None
-    assert nq.lib().nuq_panel_plan(0, 64, 256, 100, 144, 256, 0, (ctypes.c_uint64 * 9)()) == 0
+    assert nq.lib().nuq_panel_plan(0, 64, 256, 100, 144, 256, 0, 256, (ctypes.c_uint64 * 9)()) == 0
     assert plan(12, 64, 256, 100, 0, in_stride=1 << 23) is None
     assert plan(12, 64, 256, 100, 0, in_stride=1 << 22) is not None
 
