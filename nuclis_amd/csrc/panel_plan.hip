@@ -83,9 +83,9 @@ static const PanelCost PANEL_COST[5][PANEL_SHAPE_COUNT] = {
 };
 
 struct PanelShape {
-    uint8_t tg, rg, wr, wk;
+    uint8_t tg, rg, wr, wk, depth;
 };
-#define NUQ_PANEL_ROW(I, T, R, W, K, D) {T, R, W, K},
+#define NUQ_PANEL_ROW(I, T, R, W, K, D) {T, R, W, K, D},
 static const PanelShape PANEL_SHAPES[PANEL_SHAPE_COUNT] = {NUQ_PANEL_SHAPES(NUQ_PANEL_ROW)};
 #undef NUQ_PANEL_ROW
 
@@ -232,6 +232,32 @@ hipError_t launch_panel(hipStream_t s, uint32_t encoding, const PanelArgs &a, co
     hipLaunchKernelGGL(panel_reduce_kernel, dim3(p.tail * (bm * bn / 1024)), dim3(256), 0, s, work, a.y, a.out_stride,
                        a.rows, a.tokens, bm, bn, p.full, p.splits, PANEL_GROUP);
     return hipGetLastError();
+}
+
+// For checks: the fields of shape i (TG, RG, WR, WK, DEPTH), 0 past the last
+// shape, and one product on a given plan.
+extern "C" int nuq_panel_shape(uint32_t i, uint32_t out[5]) {
+    if (i >= (uint32_t)PANEL_SHAPE_COUNT) return 0;
+    const PanelShape &s = PANEL_SHAPES[i];
+    const uint32_t v[5] = {s.tg, s.rg, s.wr, s.wk, s.depth};
+    std::copy(v, v + 5, out);
+    return 1;
+}
+
+extern "C" int nuq_panel_run(void *stream, uint32_t encoding, const void *w, uint64_t stride, uint32_t rows,
+                             uint32_t columns, const void *x, uint64_t in_stride, void *y, uint64_t out_stride,
+                             uint32_t tokens, uint32_t shape, uint32_t full, uint32_t tail, uint32_t splits,
+                             void *work) {
+    if (shape >= (uint32_t)PANEL_SHAPE_COUNT || splits == 0 || tokens == 0 || columns % 256 != 0)
+        return (int)hipErrorInvalidValue;
+    const PanelShape &sh = PANEL_SHAPES[shape];
+    const uint32_t bm = 32 * sh.tg, bn = 32 * sh.rg * sh.wr;
+    if (full + tail != (tokens + bm - 1) / bm * ((rows + bn - 1) / bn) || splits * sh.wk > columns / 256)
+        return (int)hipErrorInvalidValue;
+    const PanelPlan p{(int)shape, full, tail, splits, (uint64_t)tail * splits * bm * bn, 0.f};
+    const PanelArgs a{(const uint8_t *)w, stride, rows, columns, (const _Float16 *)x, in_stride, (float *)y, out_stride,
+                      tokens};
+    return (int)launch_panel((hipStream_t)stream, encoding, a, p, (float *)work);
 }
 
 // Eight values a thread, rounded to nearest even as the tiles' own conversion.

@@ -15,20 +15,9 @@ from tests.gpu_util import F16_K, check_close, mass, to_gpu
 
 pytestmark = pytest.mark.gpu
 
-# NUQ_PANEL_SHAPES (nuclis_amd/csrc/panel.h): TG, RG, WR, WK, DEPTH
+# TG, RG, WR, WK, DEPTH of the library's shapes (test_shape_table)
 SHAPES = [(1, 1, 4, 1, 4), (1, 1, 2, 4, 2), (2, 1, 2, 2, 2), (3, 1, 4, 2, 2), (4, 1, 4, 2, 2),
           (4, 1, 2, 2, 2), (4, 1, 4, 1, 2), (4, 2, 4, 1, 2), (6, 2, 4, 1, 2), (8, 2, 4, 1, 2)]
-
-
-class Plan(ctypes.Structure):
-    _fields_ = [("shape", ctypes.c_int), ("full", ctypes.c_uint32), ("tail", ctypes.c_uint32),
-                ("splits", ctypes.c_uint32), ("work_floats", ctypes.c_uint64), ("cost", ctypes.c_float)]
-
-
-class Args(ctypes.Structure):
-    _fields_ = [("w", ctypes.c_void_p), ("stride", ctypes.c_uint64), ("rows", ctypes.c_uint32),
-                ("columns", ctypes.c_uint32), ("x", ctypes.c_void_p), ("in_stride", ctypes.c_uint64),
-                ("y", ctypes.c_void_p), ("out_stride", ctypes.c_uint64), ("tokens", ctypes.c_uint32)]
 
 
 @pytest.fixture(scope="module")
@@ -40,12 +29,22 @@ def backend():
     b.close()
 
 
-def launch(encoding, args, plan, work):
+def launch(encoding, w, x, columns, y, shape, full, tail, splits, work):
+    """One product on the given plan: w [rows][bytes], x [tokens][stride], y
+    [tokens][stride], all on the GPU; rows come with `w`, tokens with `x`."""
     import torch
-    f = nq.lib()._ZN3nuq12launch_panelEP12ihipStream_tjRKNS_9PanelArgsERKNS_9PanelPlanEPf
-    f.restype = ctypes.c_int
-    f.argtypes = [ctypes.c_void_p, ctypes.c_uint32, ctypes.POINTER(Args), ctypes.POINTER(Plan), ctypes.c_void_p]
-    return f(torch.cuda.current_stream().cuda_stream, encoding, ctypes.byref(args), ctypes.byref(plan), work)
+    f, u32, u64, vp = nq.lib().nuq_panel_run, ctypes.c_uint32, ctypes.c_uint64, ctypes.c_void_p
+    f.argtypes = [vp, u32, vp, u64, u32, u32, vp, u64, vp, u64, u32, u32, u32, u32, u32, vp]
+    return f(torch.cuda.current_stream().cuda_stream, encoding, w.data_ptr(), w.shape[1], w.shape[0], columns,
+             x.data_ptr(), x.shape[1], y.data_ptr(), y.shape[1], x.shape[0], shape, full, tail, splits, work.data_ptr())
+
+
+def test_shape_table(backend):
+    out = (ctypes.c_uint32 * 5)()
+    table = []
+    while nq.lib().nuq_panel_shape(len(table), out):
+        table.append(tuple(out))
+    assert table == SHAPES
 
 
 @pytest.mark.parametrize("shape", range(len(SHAPES)))
@@ -67,8 +66,7 @@ def test_every_shape_matches_oracle(backend, encoding, shape):
     work = torch.empty(tiles * 2 * bm * bn, device="cuda")
     for full, tail, splits in ((tiles, 0, 1), (0, tiles, 2), (tiles - 1, 1, 2)):
         y = torch.full((tokens, out_stride), np.nan, device="cuda")
-        args = Args(wg.data_ptr(), w.shape[1], rows, columns, xg.data_ptr(), in_stride, y.data_ptr(), out_stride, tokens)
-        assert launch(encoding, args, Plan(shape, full, tail, splits, 0, 0.0), work.data_ptr()) == 0
+        assert launch(encoding, wg, xg, columns, y, shape, full, tail, splits, work) == 0
         torch.cuda.synchronize()
         got = y.cpu().numpy()
         assert np.isnan(got[:, rows:]).all() and np.isfinite(got[:, :rows]).all()
@@ -84,9 +82,8 @@ def run_shape(encoding, shape, w, x, splits=1):
     tiles = -(-tokens // bm) * -(-rows // bn)
     wg, xg, y = to_gpu(w), to_gpu(x), torch.full((tokens, rows), float("nan"), device="cuda")
     work = torch.empty(tiles * splits * bm * bn, device="cuda")
-    args = Args(wg.data_ptr(), w.shape[1], rows, columns, xg.data_ptr(), columns, y.data_ptr(), rows, tokens)
-    plan = Plan(shape, tiles, 0, 1, 0, 0.0) if splits == 1 else Plan(shape, 0, tiles, splits, 0, 0.0)
-    assert launch(encoding, args, plan, work.data_ptr()) == 0
+    assert launch(encoding, wg, xg, columns, y, shape, tiles if splits == 1 else 0, 0 if splits == 1 else tiles, splits,
+                  work) == 0
     torch.cuda.synchronize()
     return y.cpu().numpy()
 
@@ -194,8 +191,7 @@ def test_partial_sums_of_any_split_count(backend, splits):
     x = gaussian(42, (tokens, columns)).astype(np.float16)
     wg, xg = to_gpu(w), to_gpu(x)
     work, y = torch.empty(4 * splits * 32 * 128, device="cuda"), torch.full((tokens, rows), np.nan, device="cuda")
-    args = Args(wg.data_ptr(), w.shape[1], rows, columns, xg.data_ptr(), columns, y.data_ptr(), rows, tokens)
-    assert launch(14, args, Plan(0, 0, 4, splits, 0, 0.0), work.data_ptr()) == 0
+    assert launch(14, wg, xg, columns, y, 0, 0, 4, splits, work) == 0
     torch.cuda.synchronize()
     xr = x.astype(np.float32)
     check_close(y.cpu().numpy(), orc.matmul(14, rows, columns, w, xr), mass(14, w, rows, columns, xr), F16_K,
@@ -203,9 +199,10 @@ def test_partial_sums_of_any_split_count(backend, splits):
 
 
 @pytest.mark.parametrize("encoding,rows,columns,tokens", [(12, 1032, 512, 77), (14, 520, 2304, 300), (8, 4104, 2048, 260),
-                                                          (8, 264, 320, 40), (23, 8192, 4096, 8)])
+                                                          (8, 264, 320, 40), (23, 1024, 32768, 8)])
 def test_f32_activations_equal_their_f16_rounding(backend, encoding, rows, columns, tokens):
-    """The tiles round F32 activations to f16: the same bits as f16 input."""
+    """The tiles round F32 activations to f16: the same bits as f16 input (where
+    both kinds take the same tile)."""
     import torch
     w = to_gpu(nq.quantize(encoding, gaussian(3, (rows, columns), 0.02)))
     m = nq.Matrix(encoding, rows, columns, w)

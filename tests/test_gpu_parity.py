@@ -311,6 +311,27 @@ def test_streamed_verify_matches_oracle(backend, encoding, rows, columns, tokens
     check_close(out.cpu().numpy(), want, mass(encoding, w, rows, columns, xref), k, "verify")
 
 
+@pytest.mark.parametrize("encoding", [12, 13])
+@pytest.mark.parametrize("columns", [24832, 25856, 32768])
+def test_streamed_verify_of_many_ranges(backend, encoding, columns):
+    """Rows of 97, 101 and 128 blocks run as 5 to 7 K ranges, whose partial sums
+    are added four at a time: f16 tokens on the verify tile, F32 tokens in the
+    three-part form."""
+    import torch
+    rows = 40
+    w = quantized(encoding, rows, columns, 33)
+    m = nq.Matrix(encoding, rows, columns, to_gpu(w))
+    for tokens, f16 in ((8, True), (3, False)):
+        x = gaussian(34, (tokens, columns))
+        xr = x.astype(np.float16).astype(np.float32) if f16 else x
+        y = torch.full((tokens, rows), np.nan, device="cuda")
+        backend.matmul(m, to_gpu(x.astype(np.float16) if f16 else x), columns, y, rows, tokens)
+        backend.sync()
+        # exact products either way: the F32 bound
+        check_close(y.cpu().numpy(), orc.matmul(encoding, rows, columns, w, xr), mass(encoding, w, rows, columns, xr), F32_K,
+                    f"verify-ranges {encoding} {columns} T={tokens}")
+
+
 @pytest.mark.parametrize("pad", [8, 64])
 def test_streamed_verify_strided_activations(backend, pad):
     """f16 activation rows `pad` halves longer than K (staged through LDS in
