@@ -68,7 +68,7 @@ __device__ __forceinline__ half2v subnormal_bytes(uint32_t t) {
 // byte goes into the mantissa of 1024.0, whose ulp is 1), whose bias the F32
 // addend takes out. The addend is exact (the scale has at most 18 bits, the
 // bias 6), but infinite with the scale: infinite scales are replaced
-// (overflowing) before.
+// (overflowing) before, and Q6_K rows with a NaN weight found after the loop.
 constexpr uint32_t F16_1024 = 0x64006400u;
 template <uint32_t M>
 __device__ __forceinline__ half2v biased(uint32_t t) {
@@ -236,7 +236,12 @@ struct PanelRaw<14> {
     u32x4 ql[4], qh[2], sc;
     uint32_t d16;
     float d, mul0, add0, mul1, add1;
-    __device__ __forceinline__ void open() { d = half_bits(d16); }
+    uint64_t inf = 0;  // lanes that met an infinite d
+    __device__ __forceinline__ void open() {
+        d = half_bits(d16);
+        inf |= __builtin_amdgcn_ballot_w64(fabsf(d) == INFINITY);
+        d = overflowing(d);
+    }
     __device__ static uint32_t src(uint32_t c) { return c < 13 ? 16 * c : 194; }
     __device__ static uint32_t chunk_of(uint32_t c, uint32_t part) { return (c & 1) * 4 + part * 2 + (c >> 1); }
     __device__ __forceinline__ void read(const uint8_t *unit, const uint8_t *, uint32_t part) {
@@ -271,20 +276,22 @@ struct PanelRaw<14> {
         }
         return f;
     }
-    // An infinite d, from the row's image: NaN if any weight of the block is (a
-    // zero code or scale; its other weights only meet outputs that are NaN with
-    // it), else a value that overflows. A rolled loop: unrolled over the
-    // registers it would cost the main loop half its waves.
-    __device__ __forceinline__ void settle(const uint8_t *unit) {
-        if (fabsf(d) != INFINITY) return;
-        bool zero = false;
+    // Whether a weight of the row's blocks [b0, b1) is NaN: an infinite d times
+    // a zero code or scale.
+    __device__ static bool nan_weight(const uint8_t *row, uint32_t b0, uint32_t b1) {
+        bool nan = false;
 #pragma unroll 1
-        for (uint32_t k = 0; k < 128; ++k) {
-            const uint32_t l = unit[k], h = unit[128 + (k >> 6) * 32 + (k & 31)] >> (2 * ((k >> 5) & 1));
-            zero = zero || ((l & 15u) | (h & 3u) << 4) == 32u || (l >> 4 | ((h >> 4) & 3u) << 4) == 32u ||
-                   unit[192 + (k & 15)] == 0;
+        for (uint32_t b = b0; b < b1; ++b) {
+            const uint8_t *blk = row + (uint64_t)b * BYTES;
+            if ((load_u16_bytes(blk + 208) & 0x7fffu) != 0x7c00u) continue;
+#pragma unroll 1
+            for (uint32_t k = 0; k < 128; ++k) {
+                const uint32_t l = blk[k], h = blk[128 + (k >> 6) * 32 + (k & 31)] >> (2 * ((k >> 5) & 1));
+                nan = nan || ((l & 15u) | (h & 3u) << 4) == 32u || (l >> 4 | ((h >> 4) & 3u) << 4) == 32u ||
+                      blk[192 + (k & 15)] == 0;
+            }
         }
-        d = zero ? NAN : overflowing(d);
+        return nan;
     }
 };
 
@@ -570,21 +577,6 @@ __global__ void __launch_bounds__(64 * WR * WK, (panel_waves<ENC, TG, RG, WR, WK
         if constexpr (FENCE) __builtin_amdgcn_sched_barrier(0);                                                \
     }
     for (uint32_t ks = ks0; ks < ks1; ks += 4) {
-        // an infinite Q6_K scale in the unit just opened: a wave-uniform
-        // branch where the loop turns, outside the schedule of the steps
-        if constexpr (ENC == 14) {
-            bool inf = false;
-#pragma unroll
-            for (int g = 0; g < RG; ++g) inf = inf || fabsf(raw[g].d) == INFINITY;
-            if (__builtin_amdgcn_ballot_w64(inf) != 0) {
-#pragma unroll
-                for (int g = 0; g < RG; ++g) {
-                    raw[g].settle(image + g * 32 * ROWB);
-                    raw[g].template setup<0>(part);
-                    fb[0][g] = raw[g].template chunk<0, 0>();
-                }
-            }
-        }
         PN_STEP(0)
         PN_STEP(1)
         PN_STEP(2)
@@ -597,6 +589,22 @@ __global__ void __launch_bounds__(64 * WR * WK, (panel_waves<ENC, TG, RG, WR, WK
 #undef PN_RAW
 #undef PN_READ
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");  // no copy into LDS outlives the workgroup
+
+    // Infinite Q6_K scales took part as values that overflow, with which a zero
+    // code or scale gives 0: rows that have one there are NaN. (A scan of those
+    // rows after the loop: a branch in it costs 1 % at 8 tokens.)
+    if constexpr (ENC == 14) {
+#pragma unroll
+        for (int g = 0; g < RG; ++g)
+            if (raw[g].inf >> lane & 1) {
+                const uint32_t r = min(wr * (32 * RG) + g * 32 + l32, rows - 1 - n_base);
+                if (Raw::nan_weight(wt + (uint64_t)r * stride, ks0 / 4, ks1 / 4))
+#pragma unroll
+                    for (int t = 0; t < TG; ++t)
+#pragma unroll
+                        for (int q = 0; q < 16; ++q) acc[t][g][q] = NAN;
+            }
+    }
 
     // D layout: lane l32 holds weight row n; register r token 8 (r / 4) + 4 part + r % 4
     float *mine = split_k ? work + (uint64_t)((tile - full) * splits + split) * (BM * BN) : nullptr;

@@ -141,7 +141,7 @@ def test_infinite_scales_keep_the_weights_signs(backend, encoding, shape):
     """A block of infinite scale: +-Inf for codes of one sign, NaN for a zero
     code (rows 1 mod 4) and for a scale of zero (rows 2 mod 4); rows 0 mod 4
     are finite."""
-    rows, tokens, columns = 200, 40, 256 * max(2, SHAPES[shape][3])
+    rows, tokens, columns = 200, 40, 512 * SHAPES[shape][3]
     values, _ = nq.LAYOUT[encoding]
     b = blocks(encoding, rows, columns, 81)
     sick = np.arange(rows) % 4 != 0
@@ -177,9 +177,10 @@ def test_infinite_scales_keep_the_weights_signs(backend, encoding, shape):
         want = (dec[None] * x.astype(np.float64)[:, None, :]).sum(-1)
     assert np.isposinf(want).any() and np.isneginf(want).any() and np.isnan(want).any()
     assert np.isfinite(want[:, ~sick]).all()
-    got = run_shape(encoding, shape, w, x)
-    for cls in (np.isnan, np.isposinf, np.isneginf):
-        assert np.array_equal(cls(got), cls(want)), cls.__name__
+    for splits in (1, 2):
+        got = run_shape(encoding, shape, w, x, splits)
+        for cls in (np.isnan, np.isposinf, np.isneginf):
+            assert np.array_equal(cls(got), cls(want)), (cls.__name__, splits)
 
 
 @pytest.mark.parametrize("splits", [2, 4, 5, 6, 9, 11])
