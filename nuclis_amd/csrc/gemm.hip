@@ -2357,7 +2357,7 @@ uint64_t verify_workspace_floats(uint32_t encoding, uint32_t rows, uint32_t colu
 // Predicted time (us) of Q8_0 on the prefill tile with f16 activations: 3.6 us
 // a round of a tile per CU, 8.54 us a 256-column block of a round, 0.4 us per MB of
 // split partial sums. Fitted to the times from 64 to 4096 tokens on 17408 x
-// 5120, 5120 x 17408 and 4096 x 4096 (6 % rms).
+// 5120, 5120 x 17408 and 4096 x 4096 (6 % rms; profiles/fit_costs.py).
 static float prefill_cost(uint32_t rows, uint32_t columns, uint32_t tokens, uint64_t max_floats, uint32_t cus) {
     const uint32_t tiles = ((tokens + PF_BM - 1) / PF_BM) * ((rows + PF_BN - 1) / PF_BN), nb = columns / 256;
     uint32_t full, tail, splits;
@@ -2372,8 +2372,8 @@ static float prefill_cost(uint32_t rows, uint32_t columns, uint32_t tokens, uint
 // a + (b + c tokens) us per 256-column block of 16 rows on the busiest CU, so it
 // wins where its row groups fill the CUs in whole rounds (4096 rows: one each);
 // the panel model is low by the last two factors for whole and split tiles at
-// these tokens. Fitted to 172 timings each (43 matrices of 2^25 weights and more, 4 to
-// 16 tokens): the choice takes 1.004 (Q8_0), 1.009 (Q6_K) and 1.006 (IQ4_XS)
+// these tokens. Fitted to 172 timings each (matrices of 2^25 weights and more, 4
+// to 16 tokens; profiles/fit_costs.py): the choice takes 1.004 (Q8_0), 1.008 (Q6_K) and 1.006 (IQ4_XS)
 // of the better tile's time on average and 1.15 at most over the verify tile's,
 // where the panel tile for all took up to 1.44, 1.37 and 1.72 (IQ4_XS 4096 x
 // 9216 at 4 tokens 18.7 us against 10.8).

@@ -11,10 +11,10 @@ namespace nuq {
 // (its LDS and registers); a round of the grid with q workgroups on the busiest
 // CU takes a + n (b + c (q - 1)) us, n the 256-column blocks of a wave set. A
 // split adds r0 us and r1 us per MB of partial sums. Fitted per encoding and
-// shape to 11,600 timings on MI355X (six matrices from 1024 x 5120 to 17408 x
-// 5120, 4 to 4096 tokens): relative error 5-9 % rms, and the plan chosen takes
-// 1.02 of the best measured plan's time on average (at most 1.2). Encodings
-// 8, 12, 13, 14, 23.
+// shape to 11,421 timings on MI355X (six matrices from 1024 x 5120 to 17408 x
+// 5120, 4 to 4096 tokens; profiles/fit_costs.py prints this table from them):
+// relative error 5-10 % rms, and the plan chosen takes 1.02 of the best measured
+// plan's time on average (at most 1.32). Encodings 8, 12, 13, 14, 23.
 struct PanelCost {
     uint8_t occ;
     float a, b, c, r0, r1;
