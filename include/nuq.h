@@ -93,14 +93,15 @@ void nuq_destroy(nuq_context *ctx);
 int nuq_set_stream(nuq_context *ctx, void *stream);
 /* The context's device workspace (verify K-range partials, split partial
  * tiles, the f16 copy of F32 activations, a mixed SiLU pair's second GEMV) is
- * allocated on the first call that wants it and grown as needed; nuq_create allocates none. A call that would
- * grow it while a graph capture is active takes its no-workspace route
- * instead (same products). A workspace that a captured call used is never
+ * allocated on the first call that wants it and grown by powers of two (4 to
+ * 512 MiB; nuq_reserve_workspace exactly); nuq_create allocates none. A call
+ * that would grow it while a graph capture is active takes its no-workspace
+ * route instead (same products). A workspace that a captured call used is never
  * freed on growth: it stays allocated until nuq_destroy, so graphs captured
  * earlier keep replaying into valid memory (they must not replay after
  * nuq_destroy). Callers that capture graphs may reserve it beforehand, so it
- * never grows after a capture. No counterpart in the reference (Metal buffers are created per
- * use, backends/metal/root.zig:62-86). */
+ * never grows after a capture. No counterpart in the reference (Metal buffers
+ * are created per use, backends/metal/root.zig:62-86). */
 int nuq_reserve_workspace(nuq_context *ctx, uint64_t bytes);
 /* Bytes of workspace the context currently holds. */
 uint64_t nuq_workspace_bytes(const nuq_context *ctx);
@@ -156,10 +157,10 @@ int nuq_matvec_segments(nuq_context *ctx, const nuq_segment *segments, uint32_t 
 #define NUQ_NOALLOC_MAX_PAIR_ROWS (1u << 20)
 /* nuq_matvec_segments without any allocation: no counterpart in the
  * reference. For callers that cannot allocate device memory (code under HIP
- * graph capture, tight serving loops). The SiLU pair's second GEMV goes to a
- * fixed 4 MiB scratch array in device memory, one per GPU, held until the
- * process ends, instead of the context workspace; pairs of more than
- * NUQ_NOALLOC_MAX_PAIR_ROWS rows are refused (NUQ_INVALID_SHAPE) before
+ * graph capture, tight serving loops). The second GEMV of a SiLU pair that
+ * runs as two goes to a fixed 4 MiB scratch array in device memory, one per
+ * GPU, held until the process ends, instead of the context workspace; pairs of
+ * more than NUQ_NOALLOC_MAX_PAIR_ROWS rows are refused (NUQ_INVALID_SHAPE) before
  * anything is launched. Same validation, kernels and results as
  * nuq_matvec_segments otherwise. Every call on one GPU shares that GPU's
  * scratch: calls that overlap on one GPU (other streams, other contexts of
