@@ -111,16 +111,17 @@ bool panel_plan(uint32_t encoding, uint32_t rows, uint32_t columns, uint32_t tok
     if (256 * stride > 0xffffffffull || 256 * in_stride * 2 + 2ull * columns > 0xffffffffull) return false;
     const uint32_t nb = columns / 256;
     const uint32_t groups = (tokens + 31) / 32;
-    // shapes of more token groups than the tokens fill only add padding, and
-    // small ones decode the weights once more per token tile; rows of one
-    // block have no second K set for the three-group shape, so 65 to 96 tokens
-    // pad to four groups there
-    const uint32_t widest = nb == 1 && groups == 3 ? 4 : groups;
+    // Shapes of more token groups than the tokens fill only add padding, and
+    // small ones decode the weights once more per token tile: not considered
+    // beyond two tiles, except for rows of one block, where only the one-group
+    // shape and those of four groups and more have no second K set, and a tile
+    // is bound by its start-up (4096 x 256 at 96 tokens on one / four groups:
+    // IQ4_XS 5.5 / 12.7 us, Q4_K 5.0 / 8.1; at 200 tokens 6.0 / 14.1, 5.6 / 8.9).
     bool found = false;
     for (int i = 0; i < PANEL_SHAPE_COUNT; ++i) {
         const PanelShape &s = PANEL_SHAPES[i];
         const PanelCost &k = PANEL_COST[e][i];
-        if (s.tg > widest || (s.tg < 4 && groups > 2u * s.tg) || nb < s.wk) continue;
+        if (s.tg > groups || (s.tg < 4 && groups > 2u * s.tg && nb > 1) || nb < s.wk) continue;
         const uint32_t bm = 32 * s.tg, bn = 32 * s.rg * s.wr, cap = cus * k.occ;
         const uint64_t tiles64 = (uint64_t)((tokens + bm - 1) / bm) * ((rows + bn - 1) / bn);
         if (tiles64 > 0x7fffffffu / 32) continue;

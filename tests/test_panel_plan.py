@@ -45,6 +45,16 @@ def test_every_product_has_a_plan(encoding):
               rng.choice([0, 1 << 20, 1 << 26]))
 
 
+@pytest.mark.parametrize("encoding", [8, 12, 13, 14, 23])
+@pytest.mark.parametrize("tokens", [65, 96, 128, 200])
+def test_one_block_rows_take_tiles_of_one_group(encoding, tokens):
+    """Rows of one block leave a tile nothing but its start-up: tiles of 32
+    tokens (4096 x 256 at 96 tokens IQ4_XS 5.5 us, 12.7 in tiles of 128; 5.0
+    and 8.1 for Q4_K)."""
+    for rows in (64, 1024, 4096):
+        assert plan(encoding, rows, 256, tokens, 1 << 26)[5] == 32, rows
+
+
 @pytest.mark.parametrize("cus", [256, 128, 304])
 def test_split_tails_leave_whole_rounds(cus):
     """Where only the tiles of a partial last round are split, the whole tiles
