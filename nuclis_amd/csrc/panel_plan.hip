@@ -126,7 +126,7 @@ bool panel_plan(uint32_t encoding, uint32_t rows, uint32_t columns, uint32_t tok
         const uint64_t tiles64 = (uint64_t)((tokens + bm - 1) / bm) * ((rows + bn - 1) / bn);
         if (tiles64 > 0x7fffffffu / 32) continue;
         const uint32_t tiles = (uint32_t)tiles64;
-        const auto consider = [&](uint32_t tail, uint32_t splits) {
+        const auto consider = [&](uint32_t tail, uint32_t splits, float margin = 1.f) {
             const uint64_t floats = splits > 1 ? (uint64_t)tail * splits * bm * bn : 0;
             if (floats > max_floats) return;
             float t;
@@ -138,18 +138,27 @@ bool panel_plan(uint32_t encoding, uint32_t rows, uint32_t columns, uint32_t tok
                 t = rounds_cost(k, cus, s.wk, tiles - tail, nb) + rounds_cost(k, cus, s.wk, tail * splits, (nb + splits - 1) / splits) +
                     k.r0 + k.r1 * 4e-6f * sums * ((float)splits + 0.5f);
             }
+            t *= margin;
             if (found && t >= plan->cost) return;
             found = true;
             *plan = {i, splits > 1 ? tiles - tail : tiles, splits > 1 ? tail : 0, splits, floats, t};
         };
         consider(0, 1);
-        // all tiles split, to one to four workgroups per CU
-        if (tiles < 2 * cap)
+        // all tiles split, to one to four workgroups per CU, or as far as the
+        // blocks go where the tiles are too few for one: 64 x 17408 at 200 tokens
+        // 14.7 (Q4_K) to 15.8 us (IQ4_XS) split 24 ways, 104 and 119 in whole
+        // tiles. The model is a little low with idle CUs (Q6_K 1024 x 5120 at 128
+        // tokens 15.4 us against 13.4 on the next plan), so there a split has to
+        // win by 15 %.
+        if (tiles < 2 * cap) {
+            const uint32_t most = std::min(24u, nb / s.wk);
+            if (cus / tiles > most && most > 1) consider(tiles, most, 1.15f);
             for (uint32_t u = cus; u <= 4 * cus; u += cus)
                 for (uint32_t r = 0; r < 2; ++r) {
                     const uint32_t sp = r ? (u + tiles - 1) / tiles : u / tiles;
-                    if (sp > 1 && sp <= 24 && sp * s.wk <= nb) consider(tiles, sp);
+                    if (sp > 1 && sp <= most) consider(tiles, sp);
                 }
+        }
         // only the tiles of a partial last round split
         if (tiles > cap && tiles % cap != 0)
             for (uint32_t sp = 2; sp <= 4 && sp * s.wk <= nb; ++sp) consider(tiles % cap, sp);

@@ -326,3 +326,21 @@ def test_few_tokens_on_a_large_matrix(backend, encoding, tokens):
         backend.matmul(m, xg, columns, y, rows, tokens)
         backend.sync()
         check_close(y.cpu().numpy(), want, ms, F16_K, f"panel-few {encoding} tokens {tokens}")
+
+
+@pytest.mark.parametrize("encoding", [8, 12, 13, 14, 23])
+@pytest.mark.parametrize("rows,columns,tokens", [(8, 17408, 65), (64, 5120, 200), (136, 2304, 130)])
+def test_few_tiles_on_long_rows(backend, encoding, rows, columns, tokens):
+    """Few tiles, split as far as 24 ways or their blocks go (one or two a range)."""
+    import torch
+    print(f"[panel] enc {encoding} {rows}x{columns} tokens {tokens}", flush=True)
+    w = nq.quantize(encoding, gaussian(95, (rows, columns), 0.02))
+    m = nq.Matrix(encoding, rows, columns, to_gpu(w))
+    x = to_gpu(gaussian(96, (tokens, columns)))
+    xr = x.half().float().cpu().numpy()
+    want, ms = orc.matmul(encoding, rows, columns, w, xr), mass(encoding, w, rows, columns, xr)
+    for xg in (x, x.half()):
+        y = torch.full((tokens, rows), float("nan"), device="cuda")
+        backend.matmul(m, xg, columns, y, rows, tokens)
+        backend.sync()
+        check_close(y.cpu().numpy(), want, ms, F16_K, f"panel-few-tiles {encoding} {rows}x{columns}")

@@ -55,6 +55,17 @@ def test_one_block_rows_take_tiles_of_one_group(encoding, tokens):
         assert plan(encoding, rows, 256, tokens, 1 << 26)[5] == 32, rows
 
 
+@pytest.mark.parametrize("encoding", [8, 12, 13, 14, 23])
+def test_few_tiles_are_split(encoding):
+    """Matrices of few rows and long rows: their few tiles are split as far as
+    24 ways or the blocks go, though that leaves CUs idle (64 x 17408 at 200
+    tokens: IQ4_XS 16 us, 119 whole)."""
+    for rows, columns, least in ((64, 17408, 16), (512, 17408, 8), (64, 5120, 10), (512, 5120, 4), (8, 4096, 8)):
+        for tokens in (65, 128, 200, 512):
+            p = plan(encoding, rows, columns, tokens, 1 << 26)
+            assert p[1] == 0 and p[3] * p[7] >= least, (rows, columns, tokens, p)
+
+
 @pytest.mark.parametrize("cus", [256, 128, 304])
 def test_split_tails_leave_whole_rounds(cus):
     """Where only the tiles of a partial last round are split, the whole tiles
