@@ -2354,17 +2354,30 @@ uint64_t verify_workspace_floats(uint32_t encoding, uint32_t rows, uint32_t colu
     return (uint64_t)((nblocks + max_kb - 1) / max_kb) * tokens * rows;
 }
 
-// Predicted time (us) of Q8_0 on the prefill tile with f16 activations: 3.6 us
-// a round of a tile per CU, 8.54 us a 256-column block of a round, 0.4 us per MB of
-// split partial sums. Fitted to the times from 64 to 4096 tokens on 17408 x
-// 5120, 5120 x 17408 and 4096 x 4096 (6 % rms; profiles/fit_costs.py).
+// Predicted time (us) of Q8_0 on the prefill tile with f16 activations: 6.85 us
+// a round of a tile per CU, 6.61 us a 256-column block of a round, 0.42 us per MB of
+// split partial sums. Fitted to 109 times from 64 to 4096 tokens on matrices from
+// 64 x 1280 to 17408 x 5120 and 5120 x 17408, 256-column rows among them (8 % rms with
+// 0.1 us per MB of results, which panel_beats_prefill counts; profiles/fit_costs.py).
 static float prefill_cost(uint32_t rows, uint32_t columns, uint32_t tokens, uint64_t max_floats, uint32_t cus) {
     const uint32_t tiles = ((tokens + PF_BM - 1) / PF_BM) * ((rows + PF_BN - 1) / PF_BN), nb = columns / 256;
     uint32_t full, tail, splits;
     prefill_split_plan(tiles, columns, cus, max_floats / (PF_BM * PF_BN), &full, &tail, &splits);
     const uint32_t r1 = (full + cus - 1) / cus, r2 = (tail * splits + cus - 1) / cus;
-    return 3.6f * (r1 + r2) + 8.54f * (r1 * nb + r2 * ((nb + splits - 1) / splits)) +
-           0.4f * (float)tail * splits * (PF_BM * PF_BN * 4e-6f);
+    return 6.85f * (r1 + r2) + 6.61f * (r1 * nb + r2 * ((nb + splits - 1) / splits)) +
+           0.42f * (float)tail * splits * (PF_BM * PF_BN * 4e-6f);
+}
+
+// Whether Q8_0 runs faster on the panel tile, by its plan `p`, than on the prefill
+// tile. The panel's fitted matrices are 12 blocks wide and more, where the results
+// weigh little, so it leaves out 0.2 us per MB of them beside the prefill's: without
+// that wide matrices of short rows lost (17408 x 512 at 512 tokens 31.5 us on the
+// panel tile, 24.7 on the prefill tile; 17408 x 1280 50.0 and 41.5). The choice takes
+// 1.002 of the better tile's time on average over 109 products, at most 1.04 of the
+// prefill tile's.
+static bool panel_beats_prefill(uint32_t rows, uint32_t columns, uint32_t tokens, const PanelPlan &p,
+                                uint64_t max_floats, uint32_t cus) {
+    return p.cost + 0.2f * 4e-6f * (float)rows * (float)tokens < prefill_cost(rows, columns, tokens, max_floats, cus);
 }
 
 // Whether 4 to 16 f16 tokens of Q8_0, Q6_K or IQ4_XS run faster on the panel
@@ -2406,8 +2419,7 @@ constexpr uint64_t X16_BYTES = 256ull << 20;
 //    bytes are twice the others', and the panel tile reads them once per 128 or
 //    256 tokens of every row tile through LDS (17408 x 5120 at 4096 tokens 779
 //    us against 815, at 256 tokens 84 against 98; 4096 x 4096 at 256 tokens
-//    34.6 against 28). The panel model is a little low there, so the panel has
-//    to win by 8 %.
+//    34.6 against 28).
 //  - F32 activations are rounded to f16 in one pass first (the tiles round
 //    them anyway; Q6_K 5120 x 17408 at 1999 tokens 711 us with the rounding
 //    inside the prefill tile). Without workspace for the copy (a call
@@ -2453,8 +2465,7 @@ void plan_tile(uint32_t encoding, uint32_t rows, uint32_t columns, uint32_t toke
          panel_plan(encoding, rows, columns, short_chunk, stride, row_stride, t->panel.work_floats, cus, &t->last))) {
         const bool both = !small && t->route == TilePlan::PREFILL && encoding == 8;
         if (small && x_f16 && !panel_beats_verify(encoding, rows, columns, tokens, t->panel, cus)) return;
-        if (!both ||
-            t->panel.cost < 0.92f * prefill_cost(rows, columns, chunk, std::min(max_floats - copy, split_max), cus)) {
+        if (!both || panel_beats_prefill(rows, columns, chunk, t->panel, std::min(max_floats - copy, split_max), cus)) {
             t->route = TilePlan::PANEL;
             t->chunk = chunk;
             t->copy = copy;

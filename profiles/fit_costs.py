@@ -1,6 +1,6 @@
 """Fits the constants of the tiles' cost models to the timings beside this file
 and prints them as they stand in the sources: PANEL_COST (panel_plan.hip),
-prefill_cost and panel_beats_verify (gemm.hip), with their errors.
+prefill_cost, panel_beats_prefill and panel_beats_verify (gemm.hip), with their errors.
 
     python profiles/fit_costs.py
 
@@ -10,6 +10,9 @@ and K split that fits; `splits` 1 is none, n > 1 all tiles n ways, -n only the
 tiles of the last partial round. other_tile_us is the tile that served the shape
 otherwise (the prefill tile from 49 tokens). Taken with the panel tile's first
 decoding; the present one is within 1 % on 25 of its sizes (3 % on 3).
+
+prefill_times.csv: us of Q8_0 with f16 activations on the prefill tile and on the
+panel tile by its plan, on matrices of few rows and of short rows.
 
 few_token_times.csv: us through the public entry point on the register verify
 tile and on the panel tile by its plan, 4 to 16 tokens, matrices of at least
@@ -128,10 +131,36 @@ def panel():
             plans[enc, rows, columns, tokens].append((cost, us))
     ratio = [min(v)[1] / min(us for _, us in v) for v in plans.values()]
     print(f"chosen plan over best measured: mean {np.mean(ratio):.3f}, max {max(ratio):.2f} of {len(ratio)} products")
-    d = [(k[1:], us) for k, us in other.items() if k[0] == 8 and k[3] > 48]
-    x, err = fit([prefill_features(*k) for k, _ in d], [us for _, us in d])
-    print("prefill_cost (Q8_0): %.2f us a round, %.3f a block, %.3f a MB;" % tuple(x),
+    by_plan = {k: dict() for k in other if k[0] == 8 and k[3] > 48}
+    for (enc, shape), d in times.items():
+        for rows, columns, tokens, splits, us in d:
+            if (enc, rows, columns, tokens) in by_plan:
+                by_plan[enc, rows, columns, tokens][shape, splits] = us
+    prefill([(*k[1:], other[k], by_plan[k]) for k in by_plan])
+
+
+def prefill(known):
+    """known: rows, columns, tokens, us on the prefill tile, us by panel shape and splits"""
+    from tests.test_panel_plan import plan  # the library's own planner
+
+    d = []
+    for rows, columns, tokens, us, panels in known:
+        p = plan(8, rows, columns, tokens, 1 << 26)
+        d.append((rows, columns, tokens, us, panels.get((p[0], p[3] if p[1] == 0 or p[3] == 1 else -p[3]))))
+    for r in list(csv.reader(open(HERE / "prefill_times.csv")))[1:]:
+        d.append((*map(int, r[:3]), float(r[3]), float(r[4]) if r[4] else None))
+    results = np.array([q[0] * q[2] * 4e-6 for q in d])
+    x, err = fit(np.column_stack([[prefill_features(*q[:3]) for q in d], results]), [q[3] for q in d])
+    print("prefill_cost (Q8_0): %.2f us a round, %.2f a block, %.2f a MB of partial sums, %.2f a MB of results;" % tuple(x),
           "error rms %.3f of %d" % (math.sqrt((err**2).mean()), len(d)))
+    both = [(q, mb) for q, mb in zip(d, results) if q[4]]
+    tile, panel_us = (np.array([q[i] for q, _ in both]) for i in (3, 4))
+    cost = np.array([plan(8, *q[:3], 1 << 26)[8] / 1e3 for q, _ in both])
+    model = np.array([prefill_features(*q[:3]) @ x[:3] for q, _ in both])
+    for a in np.arange(0, 0.4, 0.1):
+        us = np.where(cost + a * np.array([mb for _, mb in both]) < model, panel_us, tile)
+        print("panel_beats_prefill with %.1f us a MB of results more: choice over better tile mean %.4f, over prefill at"
+              " most %.2f, %d products" % (a, (us / np.minimum(tile, panel_us)).mean(), (us / tile).max(), len(us)))
 
 
 def few_tokens():

@@ -123,7 +123,7 @@ MEASURED = [
     (23, 7168, 7168, 4, 17.7, 19.4), (23, 7168, 7168, 16, 21.9, 20.5),
     (23, 12288, 6144, 4, 23.5, 23.5), (23, 12288, 6144, 16, 30.8, 23.8),
 ]
-VERIFY, PANEL = 0, 1  # TilePlan::Route
+VERIFY, PANEL, PREFILL = 0, 1, 2  # TilePlan::Route
 
 
 def route(encoding, rows, columns, tokens, x_f16):
@@ -153,3 +153,27 @@ def test_few_f32_tokens_and_small_matrices(encoding):
     for e in (12, 13):
         assert route(e, 5120, 17408, 16, 0) == route(e, 5120, 17408, 48, 1) == VERIFY
         assert route(e, 5120, 17408, 49, 0) == route(e, 5120, 17408, 49, 1) == PANEL
+
+
+# rows, columns, tokens, us on the prefill tile, us on the panel tile: Q8_0 with
+# f16 activations on matrices of few rows or short rows, measured on MI355X
+MEASURED_Q8 = [
+    (64, 17408, 64, 37.7, 14.0), (64, 17408, 200, 37.6, 16.8), (64, 17408, 512, 41.7, 18.6),
+    (64, 17408, 1024, 42.8, 21.0), (512, 5120, 64, 23.2, 11.8), (512, 5120, 200, 23.7, 15.7),
+    (512, 5120, 512, 26.5, 20.6), (512, 5120, 1024, 26.9, 22.7), (4096, 256, 64, 12.1, 6.7),
+    (4096, 256, 200, 13.5, 7.2), (4096, 256, 512, 14.8, 11.0), (4096, 256, 1024, 16.2, 13.3),
+    (17408, 256, 64, 12.9, 10.1), (17408, 256, 512, 17.4, 25.7), (17408, 512, 64, 19.2, 11.6),
+    (17408, 512, 512, 24.7, 31.5), (17408, 1280, 64, 36.1, 20.4), (17408, 1280, 512, 41.5, 50.0),
+    (17408, 1280, 1024, 67.5, 83.1), (8192, 2048, 64, 31.9, 16.0), (8192, 2048, 200, 32.6, 21.9),
+    (8192, 2048, 512, 46.1, 33.8), (8192, 2048, 1024, 60.8, 53.8),
+]
+
+
+def test_q8_takes_the_faster_tile():
+    """Short rows leave the results' stores, long rows of few tiles the split:
+    Q8_0 runs on the tile that is the faster one there."""
+    for rows, columns, tokens, prefill, panel in MEASURED_Q8:
+        r = route(8, rows, columns, tokens, 1)
+        assert r in (PANEL, PREFILL)
+        chosen = panel if r == PANEL else prefill
+        assert chosen <= 1.1 * min(prefill, panel), (rows, columns, tokens, r, prefill, panel)
