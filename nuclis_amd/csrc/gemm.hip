@@ -2389,7 +2389,8 @@ static bool panel_beats_prefill(uint32_t rows, uint32_t columns, uint32_t tokens
 // to 16 tokens; profiles/fit_costs.py): the choice takes 1.004 (Q8_0), 1.008 (Q6_K) and 1.006 (IQ4_XS)
 // of the better tile's time on average and 1.15 at most over the verify tile's,
 // where the panel tile for all took up to 1.44, 1.37 and 1.72 (IQ4_XS 4096 x
-// 9216 at 4 tokens 18.7 us against 10.8).
+// 9216 at 4 tokens 18.7 us against 10.8). Of 48 timings on four more matrices one
+// was over that: Q8_0 4096 x 17408 at 4 tokens, 31.5 us against 26.3.
 static bool panel_beats_verify(uint32_t encoding, uint32_t rows, uint32_t columns, uint32_t tokens,
                                const PanelPlan &p, uint32_t cus) {
     struct {
